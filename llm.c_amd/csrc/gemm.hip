@@ -54,7 +54,6 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int BM = kGemmBM;   // 128
-constexpr int KT = 32;
 // LDS buffers per operand: three for 256-column tiles (144 KB, one
 // workgroup per CU either way), two for narrower tiles (whose workgroups
 // share a CU).
@@ -70,411 +69,8 @@ constexpr int gemm_stages(int wn) { return wn == 4 ? 3 : 2; }
 __device__ __forceinline__ void gemm_dma16(const float *g, unsigned lds) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(g), "{m0}"(lds) : "memory");
 }
-// An empty use of four fragments: keeps their registers allocated (and so
-// not reused) up to this point.
-__device__ __forceinline__ void keep_regs(floatx4 a, floatx4 b, floatx4 c, floatx4 d) {
-    asm volatile("" :: "v"(a), "v"(b), "v"(c), "v"(d));
-}
 // s_waitcnt limiting only the vector-memory count (expcnt, lgkmcnt at max).
 #define GEMM_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | 0x0F70)
-
-// One tile (m-tile mtg, n-tile nt) over the nk K slices from element kb;
-// the down projection writes its partial to slot `slot` (c + slot *
-// split_stride) and, with npieces > 0, records npieces for the tile's rows.
-// Every thread of the workgroup calls this together.
-template <int MODE, int WN>
-__device__ __forceinline__ void gemm_tile(const GemmArgs &a, float *smem, int mtg, int nt, int kb,
-                                          int nk, int slot, int npieces, float *part = nullptr) {
-    constexpr int BN = 64 * WN;
-    constexpr int ST = gemm_stages(WN);
-    // ST buffers each: A as 128 rows of 32 swizzled floats, B as
-    // (BN/16) x 2 packed 1 KB units (BN rows of 32 floats' worth).
-    float *As = smem;
-    float *Bs = smem + ST * BM * KT;
-    const int e = a.tile_expert[mtg];
-    const int row0 = a.offsets[e] + (mtg - a.tile_off[e]) * BM;
-    const int rows = min(BM, a.offsets[e + 1] - row0);
-    const int K = a.K;
-    const float *B = a.b + (size_t)e * a.N * K;
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    // Waves are dealt to the 4 SIMDs in turn, so with 8 waves SIMD s runs
-    // waves s and s + 4; wm = wave / WN makes them an upper-half and a
-    // lower-half wave.  When an expert's last tile is short, the MFMAs the
-    // lower-half wave skips leave its SIMD to the upper-half wave.
-    const int wm = wave / WN, wn = wave % WN;
-    // Valid 32-row MFMA blocks of this wave (0, 1 or 2); uniform per wave.
-    const int nmb = max(0, min(2, (rows - wm * 64 + 31) / 32));
-    const int li = lane & 31, lh = lane >> 5;
-
-    // Rows past the expert's last row reuse its last row: their accumulator
-    // rows are never stored, and every DMA lane stays in bounds.
-    // A tile = 16 units of 8 whole rows (32 floats = 128 B each), copied by
-    // LDS DMA: lane i of a unit's DMA brings row i / 8's 16-byte chunk
-    // (i % 8) ^ (row % 8), so row r's chunk c sits at r * 32 + 4 (c ^ (r % 8))
-    // floats and the fragment reads below are free of bank conflicts.
-    constexpr int AUW = (BM / 8) / (2 * WN);
-    const int wu = __builtin_amdgcn_readfirstlane(wave);   // (uniform: LDS DMA bases)
-    const unsigned lds0 = __builtin_amdgcn_readfirstlane(
-        (unsigned)(size_t)(const __attribute__((address_space(3))) float *)smem);
-    const float *a_src[AUW];
-#pragma unroll
-    for (int i = 0; i < AUW; ++i) {
-        const int r = 8 * (wu * AUW + i) + (lane >> 3);
-        const int c = (lane & 7) ^ (r & 7);
-        const int rr = min(r, rows - 1);
-        size_t src_row;
-        if (MODE == 0 || MODE == 2) src_row = (size_t)(a.perm[row0 + rr] / a.topk);
-        else           src_row = (size_t)(row0 + rr);
-        a_src[i] = a.a + src_row * K + 4 * c;
-    }
-    auto adma = [&](int k0, int buf) {
-#pragma unroll
-        for (int i = 0; i < AUW; ++i)
-            gemm_dma16(a_src[i] + k0, lds0 + 4u * (buf * BM * KT + (wu * AUW + i) * 256));
-    };
-    // B tile = (BN/16) x 2 units, copied whole by LDS DMA: wave w the units
-    // w * BUW .. in the packed unit layout (unit u at u * 256 floats).
-    constexpr int BUW = (BN / 16 * 2) / (2 * WN);
-    const float *b_src[BUW];
-#pragma unroll
-    for (int i = 0; i < BUW; ++i) {
-        const int u = wu * BUW + i, nbl = u >> 1, qbl = u & 1;
-        b_src[i] = B + ((size_t)(nt * (BN / 16) + nbl) * (K / 16) + qbl) * 256 + 4 * lane;
-    }
-    auto bdma = [&](int k0, int buf) {
-#pragma unroll
-        for (int i = 0; i < BUW; ++i)
-            gemm_dma16(b_src[i] + (size_t)16 * k0,
-                       lds0 + 4u * (ST * BM * KT + buf * BN * KT + (wu * BUW + i) * 256));
-    };
-    // Slice j of the tile into buffer j % ST.  With three buffers slice
-    // kt + 2 is issued during slice kt, so before the barrier that ends
-    // slice kt only the wave's newest NDMA transfers may still be in
-    // flight.
-    constexpr int NDMA = AUW + BUW;
-    auto dma = [&](int j, int buf) {
-        adma(kb + j * KT, buf);
-        bdma(kb + j * KT, buf);
-    };
-    auto wait_next = [&](int kt) {
-        if (ST == 3 && kt + 2 < nk) GEMM_WAIT_VMCNT(NDMA);
-        else GEMM_WAIT_VMCNT(0);
-    };
-
-    floatx16 acc[2][2];
-#pragma unroll
-    for (int m = 0; m < 2; ++m)
-#pragma unroll
-        for (int n = 0; n < 2; ++n)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.0f;
-
-    dma(0, 0);
-    if (ST == 3 && nk > 1) {
-        dma(1, 1);
-        GEMM_WAIT_VMCNT(NDMA);
-    } else {
-        GEMM_WAIT_VMCNT(0);
-    }
-    __syncthreads();
-    // Row (li) of this lane's A blocks has r % 8 = li % 8: the 16-byte chunk
-    // 4 lh + q of K step q sits at 4 ((4 lh + q) ^ (li % 8)) floats.
-    int aoff[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) aoff[q] = 4 * ((4 * lh + q) ^ (li & 7));
-    if (nmb == 2) {
-        // Set q holds quarter-step q's fragments (a0, a1 of the two 32-row
-        // blocks, b0, b1 of the two 32-column blocks).  Order per slice:
-        // read set 1, MFMAs of set 0, read set 2, MFMAs of set 1, read set 3,
-        // issue the DMA of slice kt + ST - 1, MFMAs of set 2, wait for the
-        // next slice, barrier, read the next slice's set 0, MFMAs of set 3.
-        // keep() holds set q's registers until the following quarter's
-        // MFMAs have issued: they wait on set q's results, so by then no
-        // MFMA reads set q and it can be refilled.  The DMA goes out after
-        // the slice's last fragment reads: LDS reads issued behind an LDS
-        // DMA of the same wave measured slower (the loop took 3 % longer
-        // with the DMA at the top of the slice).
-        floatx4 fa0[4], fa1[4], fb0[4], fb1[4];
-        const float *ap = As + (wm * 64 + li) * KT;
-        const float *bp = Bs + ((wn * 4 + (li >> 4)) * 2 + lh) * 256 + (li & 15) * 4;
-        auto rd = [&](auto bufc, auto qc) {
-            constexpr int buf = decltype(bufc)::value, q = decltype(qc)::value;
-            fa0[q] = *reinterpret_cast<const floatx4 *>(ap + buf * BM * KT + aoff[q]);
-            fa1[q] = *reinterpret_cast<const floatx4 *>(ap + buf * BM * KT + 32 * KT + aoff[q]);
-            fb0[q] = *reinterpret_cast<const floatx4 *>(bp + buf * BN * KT + 64 * q);
-            fb1[q] = *reinterpret_cast<const floatx4 *>(bp + buf * BN * KT + 4 * 256 + 64 * q);
-        };
-        auto mm = [&](auto qc) {
-            constexpr int q = decltype(qc)::value;
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa0[q][s], fb0[q][s], acc[0][0], 0, 0, 0);
-                acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa0[q][s], fb1[q][s], acc[0][1], 0, 0, 0);
-                acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa1[q][s], fb0[q][s], acc[1][0], 0, 0, 0);
-                acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa1[q][s], fb1[q][s], acc[1][1], 0, 0, 0);
-            }
-        };
-        auto keep = [&](auto qc) {
-            constexpr int q = decltype(qc)::value;
-            keep_regs(fa0[q], fa1[q], fb0[q], fb1[q]);
-        };
-        using Q0 = std::integral_constant<int, 0>;
-        using Q1 = std::integral_constant<int, 1>;
-        using Q2 = std::integral_constant<int, 2>;
-        using Q3 = std::integral_constant<int, 3>;
-        // One slice from LDS buffer buf (a constant, so every fragment
-        // address is a register plus an immediate offset).  The scheduling
-        // barriers keep the reads ahead of the MFMAs they overlap.
-        auto slice = [&](int kt, auto bufc) {
-            constexpr int buf = decltype(bufc)::value;
-            rd(bufc, Q1{});
-            __builtin_amdgcn_sched_barrier(0);
-            mm(Q0{});
-            keep(Q3{});
-            __builtin_amdgcn_sched_barrier(0);
-            rd(bufc, Q2{});
-            __builtin_amdgcn_sched_barrier(0);
-            mm(Q1{});
-            keep(Q0{});
-            __builtin_amdgcn_sched_barrier(0);
-            rd(bufc, Q3{});
-            __builtin_amdgcn_sched_barrier(0);
-            if (kt + ST - 1 < nk) dma(kt + ST - 1, (buf + ST - 1) % ST);
-            __builtin_amdgcn_sched_barrier(0);
-            mm(Q2{});
-            keep(Q1{});
-            __builtin_amdgcn_sched_barrier(0);
-            wait_next(kt);   // slice kt + 1 has landed
-            __syncthreads();
-            if (kt + 1 < nk) rd(std::integral_constant<int, (buf + 1) % ST>{}, Q0{});
-            __builtin_amdgcn_sched_barrier(0);
-            mm(Q3{});
-            keep(Q2{});
-            __builtin_amdgcn_sched_barrier(0);
-        };
-#pragma unroll
-        for (int q = 1; q < 4; ++q) fa0[q] = fa1[q] = fb0[q] = fb1[q] = floatx4{0.f, 0.f, 0.f, 0.f};
-        rd(Q0{}, Q0{});
-        for (int kt = 0; kt < nk; kt += ST) {
-            slice(kt, Q0{});
-            if (kt + 1 < nk) slice(kt + 1, Q1{});
-            if (ST == 3 && kt + 2 < nk) slice(kt + 2, std::integral_constant<int, 2 % ST>{});
-        }
-    } else {
-        // One 32-row block (the expert's last, short tile) or none.
-        for (int kt = 0; kt < nk; ++kt) {
-            const int buf = kt % ST;
-            // Slice kt + ST - 1 into the buffer slice kt - 1 used (free since
-            // the barrier that ended slice kt - 1), in flight meanwhile.
-            if (kt + ST - 1 < nk) dma(kt + ST - 1, (kt + ST - 1) % ST);
-            const float *as = As + buf * BM * KT + (wm * 64 + li) * KT;
-            const float *bs = Bs + buf * BN * KT + ((wn * 4 + (li >> 4)) * 2 + lh) * 256 + (li & 15) * 4;
-            if (nmb == 1) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    floatx4 a0 = *reinterpret_cast<const floatx4 *>(as + aoff[q]);
-                    floatx4 b0 = *reinterpret_cast<const floatx4 *>(bs + 64 * q);
-                    floatx4 b1 = *reinterpret_cast<const floatx4 *>(bs + 4 * 256 + 64 * q);
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[s], b0[s], acc[0][0], 0, 0, 0);
-                        acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[s], b1[s], acc[0][1], 0, 0, 0);
-                    }
-                }
-            }
-            wait_next(kt);   // slice kt + 1 has landed
-            __syncthreads();
-        }
-    }
-
-    // Accumulator layout of a 32x32 block: lane l, register r holds
-    // row 8*(r/4) + 4*(l/32) + (r%4), column l%32.
-    if (MODE != 1 && part) {
-        // A piece of a split tile: raw sums, [row][tile column].
-#pragma unroll
-        for (int m = 0; m < 2; ++m)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                int row = wm * 64 + m * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                if (row < rows)
-#pragma unroll
-                    for (int n = 0; n < 2; ++n)
-                        part[row * BN + wn * 64 + n * 32 + li] = acc[m][n][r];
-            }
-    } else if (MODE == 0) {
-        const int f = ((nt * BN + wn * 64) >> 1) + li;   // feature index
-#pragma unroll
-        for (int m = 0; m < 2; ++m)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                int row = wm * 64 + m * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                if (row < rows)
-                    a.c[(size_t)(row0 + row) * a.ldc + f] = swiglu_fast(acc[m][0][r], acc[m][1][r]);
-            }
-    } else if (MODE == 2) {
-        // Raw gate and up columns (packed order, dispatch-ordered rows) and H.
-        const int f = ((nt * BN + wn * 64) >> 1) + li;
-        const int col = nt * BN + wn * 64 + li;
-#pragma unroll
-        for (int m = 0; m < 2; ++m)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                int row = wm * 64 + m * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                if (row < rows) {
-                    const size_t p = (size_t)(row0 + row);
-                    const float g = acc[m][0][r], u = acc[m][1][r];
-                    a.c[p * a.ldc + col] = g;
-                    a.c[p * a.ldc + col + 32] = u;
-                    a.c2[p * a.ldc2 + f] = swiglu_fast(g, u);
-                }
-            }
-    } else if (MODE == 3) {
-        // acc = dH for features f = nt*BN + wn*64 + 32n + li; the gate and up
-        // values of f sit at packed columns 64(f/32) + f%32 and 32 past it,
-        // and are replaced by dG = dH u silu'(g), dU = dH silu(g).
-#pragma unroll
-        for (int m = 0; m < 2; ++m)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                int row = wm * 64 + m * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                if (row < rows) {
-                    float *gu = a.c + (size_t)(row0 + row) * a.ldc;
-#pragma unroll
-                    for (int n = 0; n < 2; ++n) {
-                        const int col = 2 * (nt * BN + wn * 64) + 64 * n + li;
-                        const float g = gu[col], u = gu[col + 32], dh = acc[m][n][r];
-                        const float sg = 1.0f / (1.0f + expf(-g));
-                        gu[col] = dh * u * fmaf(g * sg, 1.0f - sg, sg);
-                        gu[col + 32] = dh * g * sg;
-                    }
-                }
-            }
-    } else {
-        float *c = a.c + (size_t)slot * a.split_stride;
-#pragma unroll
-        for (int m = 0; m < 2; ++m)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                int row = wm * 64 + m * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                if (row < rows) {
-                    size_t dst = (size_t)a.perm[row0 + row] * a.ldc;
-#pragma unroll
-                    for (int n = 0; n < 2; ++n)
-                        c[dst + nt * BN + wn * 64 + n * 32 + li] = acc[m][n][r];
-                }
-            }
-        if (npieces > 0)
-            for (int r = tid; r < rows; r += 128 * WN)
-                a.pieces[(size_t)a.perm[row0 + r] * (a.N / BN) + nt] = npieces;
-    }
-}
-
-// The split tail of a gate/up launch: whole tiles [0, dp); r tiles left over
-// (dp .. dp + r - 1), each in s pieces; r = s = 0 when the tail is not split.
-struct TailLayout { int dp, r, s; };
-__device__ __forceinline__ TailLayout tail_layout(const GemmArgs &a, int ntiles, int nks) {
-    const int live = a.tile_off[a.E] * ntiles;
-    const int g = a.tail_groups;
-    const int r = live % g;
-    const int sp = r ? min(min(nks, 4), g / r) : 0;
-    if (sp < 2) return TailLayout{live, 0, 0};
-    return TailLayout{live - r, r, sp};
-}
-
-// Grid: the (m-tile, n-tile) pairs, times the reduction splits.  Down
-// projection in stream-K form (a.streamk): workgroup g takes units
-// [g per, (g + 1) per) of the flat list of (live tile, K slice) units, per =
-// ceil(units / grid); each tile it touches is a piece whose index within
-// the tile (0 for the workgroup holding the tile's first slice) is the
-// partial slot it writes, and piece 0 records the tile's piece count for
-// the combine.  Slots, pieces and counts follow from the live tile count
-// alone, so results are deterministic.
-template <int MODE, int WN>
-__global__ __launch_bounds__(128 * WN) void grouped_gemm_kernel(GemmArgs a) {
-    constexpr int BN = 64 * WN;
-    extern __shared__ __align__(16) float smem[];
-    const int ntiles = a.N / BN;
-    const int nks = a.K / KT;
-    if (MODE == 1 && a.streamk) {
-        const long units = (long)a.tile_off[a.E] * ntiles * nks;
-        const long per = (units + gridDim.x - 1) / gridDim.x;
-        long u = (long)blockIdx.x * per;
-        const long uend = u + per < units ? u + per : units;
-        while (u < uend) {
-            const int tile = (int)(u / nks);
-            const int k0 = (int)(u - (long)tile * nks);
-            const int k1 = (int)(k0 + (uend - u) < nks ? k0 + (uend - u) : nks);
-            const long tstart = (long)tile * nks;
-            const int first = (int)(tstart / per);   // workgroup of the tile's first slice
-            const int slot = (int)blockIdx.x - first;
-            const int npieces = (int)((tstart + nks - 1) / per) - first + 1;
-            gemm_tile<MODE, WN>(a, smem, tile / ntiles, tile % ntiles, k0 * KT, k1 - k0, slot,
-                                slot == 0 ? npieces : 0);
-            u += k1 - k0;
-        }
-        return;
-    }
-    if (MODE != 1 && a.tail_groups > 0) {
-        // Whole tiles in the grid's first dp workgroups, then the pieces of
-        // the split tail: piece s of tail tile r covers K slices
-        // [s nks / S, (s + 1) nks / S).  (Grid: the m-tile bound's tiles plus
-        // tail_groups.)
-        const TailLayout tl = tail_layout(a, ntiles, nks);
-        const int b = blockIdx.x;
-        if (b < tl.dp) {
-            gemm_tile<MODE, WN>(a, smem, b / ntiles, b % ntiles, 0, nks, 0, 0);
-            return;
-        }
-        const int j = b - tl.dp;
-        if (j >= tl.r * tl.s) return;
-        const int r = j / tl.s, sp = j - r * tl.s;
-        const int tile = tl.dp + r;
-        const int k0 = sp * nks / tl.s, k1 = (sp + 1) * nks / tl.s;
-        gemm_tile<MODE, WN>(a, smem, tile / ntiles, tile % ntiles, k0 * KT, k1 - k0, 0, 0,
-                            a.tail_part + (size_t)j * BM * BN);
-        return;
-    }
-    const int per_split = a.max_mtiles * ntiles;
-    const int ks = blockIdx.x / per_split;       // reduction split (down projection)
-    const int nt = (blockIdx.x % per_split) % ntiles;
-    int mtg = (blockIdx.x % per_split) / ntiles;
-    if (mtg >= a.tile_off[a.E]) return;
-    if (a.order) mtg = a.order[mtg];
-    const int nk = nks / a.ksplit;   // K steps of this split
-    gemm_tile<MODE, WN>(a, smem, mtg, nt, ks * nk * KT, nk, ks, 0);
-}
-
-template <int MODE, int WN>
-hipError_t launch_grouped(const GemmArgs &a, hipStream_t s) {
-    constexpr int BN = 64 * WN;
-    const size_t lds = (size_t)gemm_stages(WN) * (BM + BN) * KT * sizeof(float);
-    static bool attr_set = false;
-    if (!attr_set) {
-        hipError_t err = hipFuncSetAttribute(
-            reinterpret_cast<const void *>(&grouped_gemm_kernel<MODE, WN>),
-            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (err != hipSuccess) return err;
-        attr_set = true;
-    }
-    const int ntiles = a.N / BN;
-    dim3 grid((unsigned)(a.max_mtiles * ntiles * a.ksplit + (MODE != 1 ? a.tail_groups : 0)));
-    hipLaunchKernelGGL((grouped_gemm_kernel<MODE, WN>), grid, dim3(128 * WN), lds, s, a);
-    return hipGetLastError();
-}
-
-template <int MODE>
-hipError_t launch_mode(const GemmArgs &a, hipStream_t s) {
-    const GemmPlan pl = gemm_plan(a.N, a.K, a.max_mtiles, MODE == 1);
-    if (a.ksplit != (MODE == 1 ? pl.ksplit : 1)) return hipErrorInvalidValue;
-    switch (pl.bn) {
-        case 256: return launch_grouped<MODE, 4>(a, s);
-        case 128: return launch_grouped<MODE, 2>(a, s);
-        case 64:  return launch_grouped<MODE, 1>(a, s);
-        default:  return hipErrorInvalidValue;
-    }
-}
 
 // out[t] = sum over slots of gw * y, one FMA per slot in slot order
 // (src/transformer.c:355-358 after contraction), optionally added into out.
@@ -670,83 +266,6 @@ __global__ __launch_bounds__(256) void zero_ints_kernel(int *p, int n) {
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) p[i] = 0;
 }
 
-// Workgroup 8 r + q: rows 16 q .. 16 q + 15 of tail tile r of a launch with
-// a split tail, one thread per (row, 4 columns in each 32-column half of a
-// 64-column group).  The sums are the tile's S pieces added in piece order
-// (loads of four pieces in flight at a time); the tile engine's epilogue of
-// MODE then runs on them.
-template <int MODE>
-__global__ __launch_bounds__(512) void tail_fixup_kernel(GemmArgs a) {
-    constexpr int BN = 256;
-    const int ntiles = a.N / BN;
-    const TailLayout tl = tail_layout(a, ntiles, a.K / KT);
-    const int r = blockIdx.x >> 3;
-    if (r >= tl.r) return;
-    const int tile = tl.dp + r, mtg = tile / ntiles, nt = tile - mtg * ntiles;
-    const int e = a.tile_expert[mtg];
-    const int row0 = a.offsets[e] + (mtg - a.tile_off[e]) * BM;
-    const int rows = min(BM, a.offsets[e + 1] - row0);
-    const int row = 16 * (blockIdx.x & 7) + (threadIdx.x >> 5);
-    if (row >= rows) return;
-    const int g = (threadIdx.x >> 3) & 3, c = (threadIdx.x & 7) * 4;
-    const float *src = a.tail_part + (size_t)r * tl.s * BM * BN + row * BN + 64 * g + c;
-    constexpr size_t PS = (size_t)BM * BN;   // floats per piece
-    // v0: columns 64 g + c .., v1: 32 further (gate and up, or dH of two
-    // feature runs for MODE 3).
-    floatx4 v0 = {0.f, 0.f, 0.f, 0.f}, v1 = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < tl.s; s0 += 4) {
-        floatx4 p0[4], p1[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {   // (clamped: every load goes out together)
-            const size_t sq = (size_t)min(s0 + q, tl.s - 1) * PS;
-            p0[q] = *reinterpret_cast<const floatx4 *>(src + sq);
-            p1[q] = *reinterpret_cast<const floatx4 *>(src + sq + 32);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (s0 + q < tl.s) {
-                if (s0 + q == 0) { v0 = p0[0]; v1 = p1[0]; }
-                else { v0 += p0[q]; v1 += p1[q]; }
-            }
-    }
-    const size_t p = (size_t)(row0 + row);
-    if (MODE == 0 || MODE == 2) {
-        // Gate (v0) and up (v1) of features 128 nt + 32 g + c ..
-        floatx4 h;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) h[q] = swiglu_fast(v0[q], v1[q]);
-        if (MODE == 0) {
-            *reinterpret_cast<floatx4 *>(a.c + p * a.ldc + nt * (BN / 2) + 32 * g + c) = h;
-        } else {
-            float *gu = a.c + p * a.ldc + nt * BN + 64 * g + c;
-            *reinterpret_cast<floatx4 *>(gu) = v0;
-            *reinterpret_cast<floatx4 *>(gu + 32) = v1;
-            *reinterpret_cast<floatx4 *>(a.c2 + p * a.ldc2 + nt * (BN / 2) + 32 * g + c) = h;
-        }
-    } else {
-        // dH of features 256 nt + 64 g + 32 n + c .. (n = 0: v0, 1: v1); the
-        // gate and up values of feature f sit at packed columns
-        // 64 (f / 32) + f % 32 and 32 past it, replaced by dG and dU.
-#pragma unroll
-        for (int n = 0; n < 2; ++n) {
-            float *gu = a.c + p * a.ldc + 2 * (nt * BN + 64 * g) + 64 * n + c;
-            const floatx4 dhv = n ? v1 : v0;
-            floatx4 gv = *reinterpret_cast<const floatx4 *>(gu);
-            floatx4 uv = *reinterpret_cast<const floatx4 *>(gu + 32);
-            floatx4 dg, du;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float gq = gv[q], uq = uv[q], dh = dhv[q];
-                const float sg = 1.0f / (1.0f + expf(-gq));
-                dg[q] = dh * uq * fmaf(gq * sg, 1.0f - sg, sg);
-                du[q] = dh * gq * sg;
-            }
-            *reinterpret_cast<floatx4 *>(gu) = dg;
-            *reinterpret_cast<floatx4 *>(gu + 32) = du;
-        }
-    }
-}
-
 // The short-first m-tile order: thread t takes experts [t EPT, (t + 1)
 // EPT); the count of short last m-tiles before each expert comes from a
 // workgroup scan (wave shuffles, then the wave totals).
@@ -799,141 +318,12 @@ __global__ __launch_bounds__(kOrderThreads) void short_first_order_kernel(const 
 
 }  // namespace
 
-// Compute units of the current device (cached; 256 on MI355X).
-int device_cus() {
-    static int cus = 0;
-    if (cus <= 0) {
-        int dev = 0, n = 0;
-        cus = hipGetDevice(&dev) == hipSuccess &&
-                      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) ==
-                          hipSuccess && n > 0
-                  ? n : 256;
-    }
-    return cus;
-}
-
-GemmPlan gemm_plan(int N, int K, int max_mtiles, bool allow_split) {
-    GemmPlan p{0, 1};
-    if (N % 256 == 0) p.bn = 256;
-    else if (N % 128 == 0) p.bn = 128;
-    else if (N % 64 == 0) p.bn = 64;
-    else return p;
-    if (allow_split) {
-        // Down projection: the widest tile, and the reduction split (its
-        // partials are added by the combine) until the workgroups cover the
-        // CUs once: blocks of 256 columns hold a CU each, narrower ones share
-        // it 2 or 3 ways.  A split keeps >= 512 reduction elements (16 LDS
-        // slices) unless the grid is tiny.  Measured at T=4096, d=512,
-        // F=2048, E=8: no split 0.568 ms per layer, 2 splits 0.489, 4 0.501.
-        const long slots = (long)device_cus() * (p.bn == 256 ? 1 : p.bn == 128 ? 2 : 3);
-        const long blocks = (long)max_mtiles * (N / p.bn);
-        const int min_k = blocks * 4 < slots ? 128 : 512;
-        while (p.ksplit < 4 && blocks * p.ksplit < slots && K % (2 * p.ksplit * KT) == 0 &&
-               K / (2 * p.ksplit) >= min_k)
-            p.ksplit *= 2;
-        return p;
-    }
-    // Without a split: waves in flight for tile width bn (bn / 32 waves per
-    // workgroup); aim for ~4 per SIMD.  Wider tiles reuse each loaded tile
-    // across more waves, so they shrink only to 128 columns, and only tiny
-    // grids go to 64.
-    constexpr size_t kTarget = 1024;
-    auto waves = [&](int bn) { return (size_t)max_mtiles * (N / bn) * (bn / 32); };
-    while (p.bn > 128 && waves(p.bn) < kTarget) p.bn /= 2;
-    if (p.bn > 64 && waves(p.bn) < kTarget / 4 && N % 64 == 0) p.bn = 64;
-    return p;
-}
-
-DownPlan down_plan(int N, int K, int max_mtiles, size_t n) {
-    const GemmPlan g = gemm_plan(N, K, max_mtiles, true);
-    DownPlan p{g.bn, g.ksplit, 0, 0};
-    if (g.bn != 256 || K % KT) return p;
-    // Stream-K when the tiles make fewer than ~4 rounds of one workgroup per
-    // CU: every CU gets the same number of K slices, where whole tiles (or
-    // tiles split a fixed 2 or 4 ways) leave a partial last round.
-    const long cus = device_cus();
-    const long tiles_max = (long)max_mtiles * (N / 256);
-    if (tiles_max >= 4 * cus) return p;
-    const long nks = K / KT;
-    // The fewest live tiles n rows can make (all rows in full m-tiles) set
-    // the shortest run per workgroup, hence the most pieces a tile can have.
-    const long tiles_min = (long)((n + BM - 1) / BM) * (N / 256);
-    const long units_min = tiles_min * nks;
-    // At least 4 slices per workgroup on small problems.
-    const long groups = std::max(1L, std::min(cus, units_min / 4));
-    const long per_min = (units_min + groups - 1) / groups;
-    p.streamk = 1;
-    p.groups = (int)groups;
-    p.slots = (int)((nks - 1 + per_min - 1) / per_min + 1);
-    return p;
-}
-
-int gateup_tail_groups(int N, int K, int max_mtiles) {
-    const GemmPlan g = gemm_plan(N, K, max_mtiles, false);
-    const long cus = device_cus();
-    if (g.bn != 256 || K % KT || K / KT < 2 || (long)max_mtiles * (N / 256) >= 4 * cus) return 0;
-    return (int)cus;
-}
-
-hipError_t launch_gemm_gateup(const GemmArgs &a, hipStream_t s) {
-    if (a.tail_groups > 0 && (!a.tail_part || a.N % 256 || a.K % KT ||
-                              gemm_plan(a.N, a.K, a.max_mtiles, false).bn != 256))
-        return hipErrorInvalidValue;
-    return launch_mode<0>(a, s);
-}
-
-hipError_t launch_tail_fixup(const GemmArgs &a, int mode, hipStream_t s) {
-    if (a.tail_groups <= 0) return hipSuccess;
-    if (!a.tail_part || a.N % 256 || a.ldc % 4 || (mode == 2 && a.ldc2 % 4)) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)a.tail_groups * 8);
-    switch (mode) {
-        case 0: hipLaunchKernelGGL(tail_fixup_kernel<0>, grid, dim3(512), 0, s, a); break;
-        case 2: hipLaunchKernelGGL(tail_fixup_kernel<2>, grid, dim3(512), 0, s, a); break;
-        case 3: hipLaunchKernelGGL(tail_fixup_kernel<3>, grid, dim3(512), 0, s, a); break;
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_gateup_fixup(const GemmArgs &a, hipStream_t s) { return launch_tail_fixup(a, 0, s); }
-hipError_t launch_gemm_down(const GemmArgs &a, hipStream_t s) {
-    if (!a.streamk) return launch_mode<1>(a, s);
-    if (!a.pieces || a.sk_groups <= 0 || a.N % 256 || a.K % KT) return hipErrorInvalidValue;
-    constexpr size_t lds = (size_t)gemm_stages(4) * (BM + 256) * KT * sizeof(float);
-    static bool attr_set = false;
-    if (!attr_set) {
-        hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(&grouped_gemm_kernel<1, 4>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (err != hipSuccess) return err;
-        attr_set = true;
-    }
-    hipLaunchKernelGGL((grouped_gemm_kernel<1, 4>), dim3((unsigned)a.sk_groups), dim3(512), lds, s, a);
-    return hipGetLastError();
-}
-
 hipError_t launch_short_first_order(const int *offsets, const int *tile_off, int E, int *order,
                                     hipStream_t s) {
     if (E <= 0 || E > 4 * kOrderThreads || !order) return hipErrorInvalidValue;
     hipLaunchKernelGGL(short_first_order_kernel, dim3(1), dim3(kOrderThreads), 0, s, offsets,
                        tile_off, E, order);
     return hipGetLastError();
-}
-
-hipError_t launch_gemm_bwd(const GemmArgs &a, int mode, hipStream_t s) {
-    if (a.ksplit != 1) return hipErrorInvalidValue;
-    const GemmPlan pl = gemm_plan(a.N, a.K, a.max_mtiles, false);
-    if (a.K % KT || (mode != 2 && mode != 3)) return hipErrorInvalidValue;
-    if (a.tail_groups > 0 && (!a.tail_part || a.N % 256 || pl.bn != 256)) return hipErrorInvalidValue;
-#define MOE_BWD_CASE(M)                                              \
-    switch (pl.bn) {                                                 \
-        case 256: return launch_grouped<M, 4>(a, s);                 \
-        case 128: return launch_grouped<M, 2>(a, s);                 \
-        case 64:  return launch_grouped<M, 1>(a, s);                 \
-        default:  return hipErrorInvalidValue;                       \
-    }
-    if (mode == 2) { MOE_BWD_CASE(2) }
-    MOE_BWD_CASE(3)
-#undef MOE_BWD_CASE
 }
 
 hipError_t launch_combine(const CombineArgs &a, hipStream_t s) {
