@@ -917,10 +917,10 @@ hipError_t launch_moe_backward(const BackwardArgs &b, hipStream_t s) {
         GemmArgs gy = g;
         gy.a = b.H; gy.b = b.wdT; gy.c = b.Y; gy.K = F; gy.N = d; gy.ldc = d;
         gy.ksplit = py.slots; gy.split_stride = nd;
-        gy.streamk = py.streamk; gy.sk_groups = py.groups; gy.pieces = b.pieces;
+        gy.streamk = py.streamk; gy.sk_groups = py.groups; gy.sk_bn = py.bn; gy.pieces = b.pieces;
         BWD_TRY(launch_gemm_down(gy, s));
         hipLaunchKernelGGL(slot_kernel, dim3(slot_grid), dim3(256), 0, s,
-                           SlotRows{b.Y, 1, py.slots, nd, py.streamk ? b.pieces : nullptr, 256},
+                           SlotRows{b.Y, 1, py.slots, nd, py.streamk ? b.pieces : nullptr, py.bn},
                            b.dout, b.gw, b.perm, k, d, (int)n, b.dgw, b.dY, b.inv);
         // dH -> dG, dU in place over GU; dXr = dGU wgu^T by slot (over Y).
         GemmArgs gh = g;
@@ -935,9 +935,9 @@ hipError_t launch_moe_backward(const BackwardArgs &b, hipStream_t s) {
         GemmArgs gx = g;
         gx.a = GU; gx.b = b.wguT; gx.c = b.Y; gx.K = 2 * F; gx.N = d; gx.ldc = d;
         gx.ksplit = px.slots; gx.split_stride = nd;
-        gx.streamk = px.streamk; gx.sk_groups = px.groups; gx.pieces = b.pieces;
+        gx.streamk = px.streamk; gx.sk_groups = px.groups; gx.sk_bn = px.bn; gx.pieces = b.pieces;
         BWD_TRY(launch_gemm_down(gx, s));
-        dXr = SlotRows{b.Y, 1, px.slots, nd, px.streamk ? b.pieces : nullptr, 256};
+        dXr = SlotRows{b.Y, 1, px.slots, nd, px.streamk ? b.pieces : nullptr, px.bn};
     } else {
         // Recompute: G, U (gathered x rows), H, Y.
         rows(T_{}, F_{}, b.x, d, b.wg, (size_t)d * F, F, b.G, d, F, 0);

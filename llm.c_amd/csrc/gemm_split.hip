@@ -234,14 +234,15 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a, char *smem, int mtg
 #undef MOE_TILE_ROWS
 }
 
-// The split tail of a gate/up launch: whole tiles [0, dp); r tiles left over
-// (dp .. dp + r - 1), each in s pieces; r = s = 0 when the tail is not split.
+// The split tail of a gate/up launch: whole tiles [0, dp), whole rounds of
+// two workgroups per CU (2 tail_groups); r tiles left over (dp .. dp + r - 1),
+// each in s pieces, one piece per CU at most; r = s = 0 when the tail is not
+// split.
 struct TailLayout { int dp, r, s; };
 __device__ __forceinline__ TailLayout tail_layout(const GemmArgs &a, int ntiles, int nks) {
     const int live = a.tile_off[a.E] * ntiles;
-    const int g = a.tail_groups;
-    const int r = live % g;
-    const int sp = r ? min(min(nks, 4), g / r) : 0;
+    const int r = live % (2 * a.tail_groups);
+    const int sp = r ? min(min(nks, 4), a.tail_groups / r) : 0;
     if (sp < 2) return TailLayout{live, 0, 0};
     return TailLayout{live - r, r, sp};
 }
@@ -326,8 +327,10 @@ hipError_t launch_mode(const GemmArgs &a, hipStream_t s) {
     const GemmPlan pl = gemm_plan(a.N, a.K, a.max_mtiles, MODE == 1);
     if (a.K % KT || a.N % 64) return hipErrorInvalidValue;
     if (MODE == 1 && a.streamk) {
-        if (!a.pieces || a.sk_groups <= 0 || a.N % 256) return hipErrorInvalidValue;
-        return launch_grouped<MODE, 1, 4>(a, s);
+        if (!a.pieces || a.sk_groups <= 0 || a.sk_bn <= 0 || a.N % a.sk_bn) return hipErrorInvalidValue;
+        if (a.sk_bn == 256) return launch_grouped<MODE, 1, 4>(a, s);
+        if (a.sk_bn == 128) return launch_grouped<MODE, 2, 2>(a, s);
+        return hipErrorInvalidValue;
     }
     if (a.ksplit != (MODE == 1 ? pl.ksplit : 1)) return hipErrorInvalidValue;
     if (MODE != 1 && a.tail_groups > 0 && (!a.tail_part || a.N % 256 || pl.bn != 256))
@@ -464,24 +467,25 @@ GemmPlan gemm_plan(int N, int K, int max_mtiles, bool allow_split) {
     return p;
 }
 
+constexpr int kSkBN = 128, kSkPerCu = 2;
 DownPlan down_plan(int N, int K, int max_mtiles, size_t n) {
     const GemmPlan g = gemm_plan(N, K, max_mtiles, true);
     DownPlan p{g.bn, g.ksplit, 0, 0};
-    if (g.bn != 256 || K % KT) return p;
-    // Stream-K when the tiles make fewer than ~4 rounds of one workgroup per
-    // CU: every CU gets the same number of K slices, where whole tiles (or
-    // tiles split a fixed 2 or 4 ways) leave a partial last round.
+    if (g.bn < 128 || N % kSkBN || K % KT) return p;
+    // Stream-K when the tiles make fewer than ~4 rounds of two workgroups per
+    // CU: every workgroup gets the same number of K slices, where whole tiles
+    // (or tiles split a fixed 2 or 4 ways) leave a partial last round.
     const long cus = device_cus();
-    const long tiles_max = (long)max_mtiles * (N / 256);
-    if (tiles_max >= 4 * cus) return p;
+    if ((long)max_mtiles * (N / 256) >= 8 * cus) return p;
     const long nks = K / KT;
     // The fewest live tiles n rows can make (all rows in full m-tiles) set
     // the shortest run per workgroup, hence the most pieces a tile can have.
-    const long tiles_min = (long)((n + BM - 1) / BM) * (N / 256);
+    const long tiles_min = (long)((n + BM - 1) / BM) * (N / kSkBN);
     const long units_min = tiles_min * nks;
     // At least 4 slices per workgroup on small problems.
-    const long groups = std::max(1L, std::min(cus, units_min / 4));
+    const long groups = std::max(1L, std::min(kSkPerCu * cus, units_min / 4));
     const long per_min = (units_min + groups - 1) / groups;
+    p.bn = kSkBN;
     p.streamk = 1;
     p.groups = (int)groups;
     p.slots = (int)((nks - 1 + per_min - 1) / per_min + 1);
@@ -491,7 +495,7 @@ DownPlan down_plan(int N, int K, int max_mtiles, size_t n) {
 int gateup_tail_groups(int N, int K, int max_mtiles) {
     const GemmPlan g = gemm_plan(N, K, max_mtiles, false);
     const long cus = device_cus();
-    if (g.bn != 256 || K % KT || K / KT < 2 || (long)max_mtiles * (N / 256) >= 4 * cus) return 0;
+    if (g.bn != 256 || K % KT || K / KT < 2 || (long)max_mtiles * (N / 256) >= 8 * cus) return 0;
     return (int)cus;
 }
 

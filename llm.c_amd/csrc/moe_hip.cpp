@@ -1237,10 +1237,10 @@ struct FwdPlan {
     bool use_decode = false, fused = false;
     bool tiny = false;      // a step of at most moe::kTinySlots assignments (decode_tiny.hip)
     int ksplit = 1;         // partial products per slot the combine adds (at most, stream-K)
-    int streamk = 0, sk_groups = 0;   // down projection in stream-K form (moe::down_plan)
+    int streamk = 0, sk_groups = 0, sk_bn = 0;   // down projection in stream-K form (moe::down_plan)
     size_t h_floats = 0;    // H [n x F] (grouped GEMMs, unfused decode)
     size_t ys_floats = 0;   // per-slot products / split-K partials
-    size_t pieces_ints = 0; // stream-K piece counts [n][d / 256]
+    size_t pieces_ints = 0; // stream-K piece counts [n][d / sk_bn]
     int gu_tail = 0;        // gate/up split tail: workgroups per round (moe::gateup_tail_groups)
     size_t gu_part_floats = 0;  // its pieces
     size_t order_ints = 0;  // the down projection's short-first m-tile order (whole tiles, >= 4 rounds)
@@ -1254,7 +1254,7 @@ struct FwdBufs {
     int *counts = nullptr, *offsets = nullptr, *tile_off = nullptr, *tile_expert = nullptr;
     int *perm = nullptr;    // [n]
     float *h = nullptr, *ys = nullptr;
-    int *pieces = nullptr;     // [n][d / 256] (stream-K down projection)
+    int *pieces = nullptr;     // [n][d / sk_bn] (stream-K down projection)
     float *gu_part = nullptr;  // gate/up split-tail pieces
     int *order = nullptr;      // [max_mtiles] m-tile order of the down projection
     int *counters = nullptr;   // kMaxCounters ints, zero between launches
@@ -1312,11 +1312,12 @@ int plan_forward(const MoeHipLayer *L, int T, FwdPlan *p, bool probs_given) {
         p->ksplit = dp.slots;
         p->streamk = dp.streamk;
         p->sk_groups = dp.groups;
-        p->pieces_ints = dp.streamk ? n * (size_t)(d / 256) : 0;
+        p->sk_bn = dp.bn;
+        p->pieces_ints = dp.streamk ? n * (size_t)(d / dp.bn) : 0;
         p->gu_tail = moe::gateup_tail_groups(2 * F, d, p->max_mtiles);
         p->gu_part_floats = (size_t)p->gu_tail * moe::kGemmBM * 256;
         if (!dp.streamk && dp.slots == 1 && dp.bn == 256 &&
-            (long)p->max_mtiles * (d / 256) >= 4L * moe::device_cus())
+            (long)p->max_mtiles * (d / 256) >= 8L * moe::device_cus())
             p->order_ints = (size_t)p->max_mtiles;
         p->h_floats = n * F;
         p->ys_floats = (size_t)p->ksplit * n * d;
@@ -1486,6 +1487,7 @@ static int run_forward(MoeHipLayer *L, const float *x, int T, float *out, float 
         dn.split_stride = n * (size_t)d;
         dn.streamk = p.streamk;
         dn.sk_groups = p.sk_groups;
+        dn.sk_bn = p.sk_bn;
         dn.pieces = b.pieces;
         if (b.order) {
             // The experts' short last m-tiles first: a CU that finishes one of
@@ -1500,7 +1502,7 @@ static int run_forward(MoeHipLayer *L, const float *x, int T, float *out, float 
     moe::CombineArgs ca{b.ys, b.gw, out, T, d, k, accumulate, p.ksplit, n * (size_t)d};
     if (p.streamk) {
         ca.pieces = b.pieces;
-        ca.pieces_cols = 256;
+        ca.pieces_cols = p.sk_bn;
     }
     HIP_TRY(moe::launch_combine(ca, s));
     if (g_timing) {
@@ -1720,7 +1722,7 @@ int moe_hip_backward_dev(MoeHipLayer *L, const float *x, int T, const float *dou
     // dgw, inv [n]; dlogits [T x E].
     const size_t nF = n * F, nd = n * d, ndh = moe::backward_dh_floats(n, d, F, E);
     const size_t ysplits = (size_t)moe::backward_slot_splits(d, F, max_mtiles, n);
-    const size_t npieces = engine && d % 256 == 0 ? n * (size_t)(d / 256) : 0;
+    const size_t npieces = engine && d % 128 == 0 ? n * (size_t)(d / 128) : 0;
     const size_t ntail = moe::backward_tail_floats(d, F, max_mtiles);
     // (the split-tail pieces last, 256-byte aligned)
     const size_t tail_off = (3 * nF + ndh + (ysplits + 1) * nd + 2 * n + (size_t)T * E + npieces +

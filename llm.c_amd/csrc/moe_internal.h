@@ -81,6 +81,7 @@ struct GemmArgs {
     // s, and pieces[row][n-tile] receives the tile's piece count.
     int streamk = 0;
     int sk_groups = 0;
+    int sk_bn = 0;       // its tile width (DownPlan::bn)
     int *pieces = nullptr;
     // Backward epilogues: mode 2 also writes H = swiglu(G, U) to c2.
     float *c2 = nullptr;
@@ -260,7 +261,7 @@ struct BackwardArgs {
     float aux_coef;
     float *G, *U, *H, *dH, *Y, *dY, *dgw, *dlogits;
     int *inv;
-    int *pieces = nullptr;   // [n][d / 256] when a down_plan is stream-K
+    int *pieces = nullptr;   // [n][d / 128] when a down_plan is stream-K
     // Split-tail pieces of the GU recompute and dH products (engine path),
     // backward_tail_floats(...) floats, or null for whole tiles only.
     float *tail_part = nullptr;
