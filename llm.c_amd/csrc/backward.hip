@@ -20,6 +20,7 @@
 // Two fp32 tiled GEMMs do the products: rows_gemm over the dispatch tile
 // schedule (one expert per 128-row tile), reduce_gemm with the reduction
 // over an expert's rows.  Every sum runs in a fixed order (deterministic).
+#include "gemm_split.h"
 #include "moe_internal.h"
 #include "moe_math.h"
 
@@ -353,170 +354,209 @@ __global__ __launch_bounds__(256) void reduce_gemm_kernel(ReduceGemm g) {
     }
 }
 
-// The same product on the matrix cores for M, N multiples of 64 WM and
-// 64 WN over the experts' row ranges: a 64 WM x 64 WN tile per workgroup,
-// NWM x NWN waves of 32 x 32 blocks of v_mfma_f32_32x32x2f32 (lane half h
-// feeds rows 2i + h of the slice).  Rows go through LDS in
-// double-buffered slices of 32, the next two slices' loads in registers
-// while the current one is multiplied; rows past the range enter LDS as zeros.  Row
-// strides of 32 mod 64 floats: the two half-waves' rows fall in disjoint
-// banks.  The larger tiles read each operand row once per 128 columns
-// instead of once per 64.
-constexpr int kMR = 32;
+// The same product on the bf16 matrix cores with split operands
+// (gemm_split.h), for M, N multiples of 64 WM and 64 WN over the experts' row
+// ranges: a 64 WM x 64 WN tile per workgroup, 2 x 2 waves of (32 WM) x
+// (32 WN).  The reduction runs over rows, so an operand piece is eight rows
+// of one column: per step of 16 rows a wave loads eight rows of 64 columns of
+// A and of B (one column per lane), splits them and stores them as three
+// planes in MFMA operand order (two LDS stages, one barrier per step).  Rows
+// are loaded kRedAhead steps ahead: a step is 0.3-0.4 us of MFMAs, a load
+// from memory 1-2 us (one step ahead the 128 x 128 tiles of T = 4096, d = 256,
+// F = 1024 took 118 us instead of 85).  The gathered rows' perm entries come a
+// step earlier still, one per lane.
+// KG = 2: two such groups of four waves take the steps in turn and the second
+// group's sums are added to the first's at the end: for grids of one tile per
+// CU, where four waves leave the splitting, the LDS traffic and the MFMAs of a
+// step one after another (dW_g, dW_u 76 -> 71 us, dW_d 59 -> 46 there; with
+// four tiles per CU, d = 512, F = 2048, it costs 5 %).
+// Bound by the MFMAs, the splitting and the LDS traffic about equally: d =
+// 512, F = 2048, 1024 rows per expert: dW_g, dW_u 235 us (146 TFLOP/s), dW_d
+// 113; on the fp32 MFMAs 348 and 169.
+constexpr int kRedAhead = 4;
 
-template <bool GATHER, int WM, int WN, int NWM, int NWN>
-__global__ __launch_bounds__(64 * NWM * NWN) void reduce_mfma_kernel(ReduceGemm g) {
-    // NWM x NWN waves, each BM x BN blocks of 32 x 32.
-    constexpr int NT = 64 * NWM * NWN, BM = 2 * WM / NWM, BN = 2 * WN / NWN;
-    static_assert(BM >= 1 && BN >= 1 && BM * NWM == 2 * WM && BN * NWN == 2 * WN, "wave layout");
-    constexpr int TM = 64 * WM, TN = 64 * WN, LDA = TM + 32, LDB = TN + 32;
-    constexpr int QA = TM / 4, QB = TN / 4;       // float4s per slice row
-    constexpr int RA = NT / QA, RB = NT / QB;     // rows per load pass
-    constexpr int PA = kMR / RA, PB = kMR / RB;   // load passes
-    // The wider tiles fill the CUs in about one round: unused rows past the
-    // slices take the LDS above half a CU's 160 KB, so that no two of these
-    // workgroups share a CU while another CU idles.
-    constexpr int kBase = 2 * kMR * (LDA + LDB) * 4, kHalf = 80 * 1024;
-    constexpr int XR = WM * WN > 1 && kBase <= kHalf ? (kHalf - kBase) / (2 * LDA * 4) + 1 : 0;
-    __shared__ __align__(16) float As[2][kMR + XR][LDA];
-    __shared__ __align__(16) float Bs[2][kMR][LDB];
-    const int e = blockIdx.z, m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
+template <bool GATHER, int WM, int WN, int KG>
+__global__ __launch_bounds__(256 * KG, 2) void reduce_split_kernel(ReduceGemm g, unsigned topk_magic,
+                                                                unsigned topk_one) {
+    using namespace split;
+    constexpr int PLANE_A = 64 * WM * 32, PLANE_B = 64 * WN * 32;   // bytes of a plane (16 rows)
+    constexpr int STAGE = 3 * (PLANE_A + PLANE_B), D = kRedAhead;
+    constexpr int SR = 16 * KG;   // rows from one step of a group to its next
+    static_assert(KG == 1 || 4 * STAGE >= WM * WN * 16384, "LDS for the second group's sums");
+    __shared__ __align__(16) char smem_all[2 * STAGE * KG];
+    const int e = blockIdx.z, m0 = blockIdx.y * 64 * WM, n0 = blockIdx.x * 64 * WN;
     const int r0 = g.offsets[e], r1 = g.offsets[e + 1];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave / NWN, wn = wave % NWN, li = lane & 31, lh = lane >> 5;
-    const int la = tid / QA, qa = 4 * (tid % QA), lb = tid / QB, qb = 4 * (tid % QB);
-    // Two register sets take the loads of the next two slices, so each load
-    // has a slice and a half of MFMAs to arrive; the perm entries (GATHER)
-    // of a slice are loaded a slice earlier still, into a set of their own
-    // (pix, by slice parity; divided when used).  Every load is issued
-    // unconditionally, rows clamped to r1 - 1 (rows past the range are
-    // zeroed when stored to LDS), so the wait counts stay exact and no load
-    // waits for a younger one.
-    fx4 ra[2][PA], rb[2][PB];
-    int pix[2][PA];
-    auto pload = [&](auto set, int r) {
+    const int lane = threadIdx.x & 63, wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = wave8 & 3, kg = wave8 >> 2;
+    char *smem = smem_all + 2 * STAGE * kg;
+    const int wm = wave >> 1, wn = wave & 1, li = lane & 31, lh = lane >> 5;
+    // What the wave stages: rows 8 half .. of each step, one 64-column group
+    // of A and of B (with 64 columns in all, two waves hold the same group
+    // and one of them stores it).
+    const int half = wave & 1, grp = wave >> 1;
+    const bool own_a = WM == 2 || grp == 0, own_b = WN == 2 || grp == (WM == 2 ? 0 : 1);
+    const float *pa = g.a + m0 + (WM == 2 ? 64 * grp : 0);   // (uniform)
+    const float *pb = g.b + n0 + (WN == 2 ? 64 * grp : 0);
+
+    float ra[D][8], rb[D][8];
+    int pix = 0;                         // lane i: perm entry of row i of the next load
+    auto token = [&](int p) -> size_t {  // perm / topk
+        return __umulhi((unsigned)p, topk_magic) + ((unsigned)p & topk_one);
+    };
+    auto load_pix = [&](int r) {
+        if (GATHER) pix = g.perm[min(r + 8 * half + (lane & 7), r1 - 1)];
+    };
+    // Rows past the range read its last row.
+    auto load = [&](auto set, int r) {
         constexpr int S = decltype(set)::value;
 #pragma unroll
-        for (int i = 0; i < PA; ++i) {
-            const int row = min(r + la + RA * i, r1 - 1);
-            pix[S][i] = GATHER ? g.perm[row] : row;
+        for (int i = 0; i < 8; ++i) {
+            const int row = min(r + 8 * half + i, r1 - 1);
+            const size_t ar = GATHER ? token(__builtin_amdgcn_readlane(pix, i)) : (size_t)row;
+            const float *qa = pa + ar * g.lda, *qb = pb + (size_t)row * g.ldb;
+            ra[S][i] = qa[(unsigned)lane];
+            rb[S][i] = qb[(unsigned)lane];
         }
+        load_pix(r + SR);
     };
-    auto gload = [&](auto set, int r) {
+    // Mask: rows past the range count as zeros.
+    auto store = [&](auto set, auto mask, int buf, int r) {
         constexpr int S = decltype(set)::value;
+        if constexpr (decltype(mask)::value)
 #pragma unroll
-        for (int i = 0; i < PA; ++i)
-            ra[S][i] = *reinterpret_cast<const fx4 *>(
-                g.a + (size_t)(GATHER ? pix[S][i] / g.topk : pix[S][i]) * g.lda + m0 + qa);
+            for (int i = 0; i < 8; ++i) {
+                const bool in = r + 8 * half + i < r1;
+                ra[S][i] = in ? ra[S][i] : 0.f;
+                rb[S][i] = in ? rb[S][i] : 0.f;
+            }
+        // Column c of a group: its 32-column block's KB, 16 bytes at c % 32
+        // of the half.
+        char *w = smem + buf * STAGE + (lane >> 5) * 1024 + 512 * half + 16 * li;
+        auto put = [&](const float (&v)[8], char *q, int plane) {
+            const Frag f = split8(fx4{v[0], v[1], v[2], v[3]}, fx4{v[4], v[5], v[6], v[7]});
 #pragma unroll
-        for (int i = 0; i < PB; ++i) {
-            const int row = min(r + lb + RB * i, r1 - 1);
-            rb[S][i] = *reinterpret_cast<const fx4 *>(g.b + (size_t)row * g.ldb + n0 + qb);
-        }
+            for (int p = 0; p < 3; ++p) *reinterpret_cast<ux4 *>(q + p * plane) = f.t[p];
+        };
+        if (own_a) put(ra[S], w + (WM == 2 ? 2048 * grp : 0), PLANE_A);
+        if (own_b) put(rb[S], w + 3 * PLANE_A + (WN == 2 ? 2048 * grp : 0), PLANE_B);
     };
-    // Store p (< PA + PB) of register set S as LDS rows of buffer buf, slice r.
-    auto sstore1 = [&](auto set, int p, int buf, int r) {
-        constexpr int S = decltype(set)::value;
-        const fx4 z = {0.f, 0.f, 0.f, 0.f};
+    fx16 acc[WM][WN];
 #pragma unroll
-        for (int i = 0; i < PA; ++i)
-            if (p == i)
-                *reinterpret_cast<fx4 *>(&As[buf][la + RA * i][qa]) =
-                    r + la + RA * i < r1 ? ra[S][i] : z;
+    for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int i = 0; i < PB; ++i)
-            if (p == PA + i)
-                *reinterpret_cast<fx4 *>(&Bs[buf][lb + RB * i][qb]) =
-                    r + lb + RB * i < r1 ? rb[S][i] : z;
-    };
-    auto sstore = [&](auto set, int buf, int r) {
-#pragma unroll
-        for (int p = 0; p < PA + PB; ++p) sstore1(set, p, buf, r);
-    };
-    fx16 acc[BM][BN];
-#pragma unroll
-    for (int i = 0; i < BM; ++i)
-#pragma unroll
-        for (int j = 0; j < BN; ++j)
+        for (int j = 0; j < WN; ++j)
 #pragma unroll
             for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
-    const int am = wm * 32 * BM + li, bn = wn * 32 * BN + li;
-    // The slice in LDS buffer buf; operands of step kk + 2 are read while
-    // step kk multiplies.  mid(p) runs after step 2 + p's MFMAs have issued
-    // (the next slice's LDS stores, one per step under the MFMAs, so that no
-    // step waits for more than one of them).
-    static_assert(PA + PB + 2 <= kMR / 2, "stores per slice");
-    auto mm = [&](int buf, auto &&mid) {
-        float av[2][BM], bv[2][BN];
-        auto rd = [&](int st, int kk) {
+    const int aoff = wm * WM * 1024 + 16 * lane, boff = 3 * PLANE_A + wn * WN * 1024 + 16 * lane;
+    // Step c of a round: multiply LDS stage c % 2, store the next step's rows
+    // (register set (c + 1) % D) and refill that set D steps on.
+    auto step = [&](auto cc, auto mask, int r) {
+        constexpr int c = decltype(cc)::value, buf = c & 1;
+        using Next = std::integral_constant<int, (c + 1) % D>;
+        ux4 fa[WM][3], fb[WN][3];
 #pragma unroll
-            for (int i = 0; i < BM; ++i) av[st][i] = As[buf][kk + lh][am + 32 * i];
+        for (int p = 0; p < 3; ++p) {
 #pragma unroll
-            for (int j = 0; j < BN; ++j) bv[st][j] = Bs[buf][kk + lh][bn + 32 * j];
-        };
-        rd(0, 0);
+            for (int i = 0; i < WM; ++i)
+                fa[i][p] = *reinterpret_cast<const ux4 *>(smem + buf * STAGE + aoff + p * PLANE_A + i * 1024);
 #pragma unroll
-        for (int kk = 0; kk < kMR; kk += 2) {
-            const int st = (kk >> 1) & 1;
-            if (kk + 2 < kMR) rd(st ^ 1, kk + 2);
-            __builtin_amdgcn_sched_barrier(0);   // (the reads go out before the MFMAs)
-#pragma unroll
-            for (int i = 0; i < BM; ++i)
-#pragma unroll
-                for (int j = 0; j < BN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[st][i], bv[st][j],
-                                                                     acc[i][j], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            const int p = kk / 2 - 2;
-            if (p >= 0 && p < PA + PB) {
-                mid(p);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            for (int j = 0; j < WN; ++j)
+                fb[j][p] = *reinterpret_cast<const ux4 *>(smem + buf * STAGE + boff + p * PLANE_B + j * 1024);
         }
-    };
-    using S0 = std::integral_constant<int, 0>;
-    using S1 = std::integral_constant<int, 1>;
-    // Slice r (parity S), held by register set S and already in LDS buffer
-    // S: the perm entries of slice r + 3 kMR go to pix set S ^ 1, register
-    // set S takes slice r + 2 kMR (perm entries in pix set S), buffer S is
-    // multiplied, and slice r + kMR (register set S ^ 1) goes to buffer
-    // S ^ 1, which every wave finished reading before the barrier that ended
-    // the previous slice.
-    auto step = [&](auto set, int r) {
-        constexpr int S = decltype(set)::value;
-        using O = std::integral_constant<int, S ^ 1>;
-        pload(O{}, r + 3 * kMR);
-        gload(set, r + 2 * kMR);
-        mm(S, [&](int p) { sstore1(O{}, p, S ^ 1, r + kMR); });
+#pragma unroll
+        for (int q = 0; q < kPairs; ++q)
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j)
+                    acc[i][j] = mma(fa[i][kPairA[q]], fb[j][kPairB[q]], acc[i][j]);
+        store(Next{}, mask, buf ^ 1, r + SR);
+        load(Next{}, r + SR * (D + 1));
         __syncthreads();
     };
     if (r0 < r1) {
-        pload(S0{}, r0);
-        pload(S1{}, r0 + kMR);
-        gload(S0{}, r0);
-        pload(S0{}, r0 + 2 * kMR);
-        gload(S1{}, r0 + kMR);
-        sstore(S0{}, 0, r0);
+        using S0 = std::integral_constant<int, 0>;
+        using S1 = std::integral_constant<int, 1>;
+        using S2 = std::integral_constant<int, 2>;
+        using S3 = std::integral_constant<int, 3>;
+        static_assert(D == 4, "register sets");
+        using Mask = std::true_type;
+        using Whole = std::false_type;
+        // (the group's own rows: step i at r + 16 kg)
+        const int o = 16 * kg;
+        load_pix(r0 + o);
+        load(S0{}, r0 + o);
+        load(S1{}, r0 + o + SR);
+        load(S2{}, r0 + o + 2 * SR);
+        load(S3{}, r0 + o + 3 * SR);
+        store(S0{}, Mask{}, 0, r0 + o);
+        load(S0{}, r0 + o + 4 * SR);
         __syncthreads();
         int r = r0;
-        for (; r + kMR < r1; r += 2 * kMR) {
-            step(S0{}, r);
-            step(S1{}, r + kMR);
+        for (; r + 5 * SR <= r1; r += 4 * SR) {   // (the rows stored are all there)
+            step(S0{}, Whole{}, r + o);
+            step(S1{}, Whole{}, r + o + SR);
+            step(S2{}, Whole{}, r + o + 2 * SR);
+            step(S3{}, Whole{}, r + o + 3 * SR);
         }
-        if (r < r1) step(S0{}, r);   // an odd last slice
+        for (; r < r1; r += 4 * SR) {
+            step(S0{}, Mask{}, r + o);
+            if (r + SR < r1) step(S1{}, Mask{}, r + o + SR);
+            if (r + 2 * SR < r1) step(S2{}, Mask{}, r + o + 2 * SR);
+            if (r + 3 * SR < r1) step(S3{}, Mask{}, r + o + 3 * SR);
+        }
+    }
+    if (KG == 2) {
+        // (every wave is past its last fragment reads: a step ends in a barrier)
+        float *x = reinterpret_cast<float *>(smem_all) + wave * (WM * WN * 1024) + lane;
+        if (kg == 1)
+#pragma unroll
+            for (int i = 0; i < WM * WN * 16; ++i) x[64 * i] = acc[i / (16 * WN)][i / 16 % WN][i % 16];
+        __syncthreads();
+        if (kg == 1) return;
+#pragma unroll
+        for (int i = 0; i < WM * WN * 16; ++i) acc[i / (16 * WN)][i / 16 % WN][i % 16] += x[64 * i];
+    }
+    // Not all finite: again as float products (gemm_split.h), rows r + lh at
+    // a time.
+    float chk = 0.f;
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) chk = fmaf(acc[i][j][q], 0.f, chk);
+    if (__ballot(!(chk == 0.f))) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                const float *ca = g.a + m0 + (wm * WM + i) * 32 + li;
+                const float *cb = g.b + n0 + (wn * WN + j) * 32 + li;
+#pragma unroll
+                for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
+#pragma unroll 1
+                for (int r = r0; r < r1; r += 2) {
+                    const int row = min(r + lh, r1 - 1);
+                    float x = ca[(GATHER ? token(g.perm[row]) : (size_t)row) * g.lda];
+                    float y = cb[(size_t)row * g.ldb];
+                    if (r + lh >= r1) x = y = 0.f;
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc[i][j], 0, 0, 0);
+                }
+            }
     }
     // Lane l, register q of a block: row 8 (q / 4) + 4 (l / 32) + q % 4,
     // column l % 32.
 #pragma unroll
-    for (int j = 0; j < BN; ++j) {
-        const int n = n0 + bn + 32 * j;
+    for (int j = 0; j < WN; ++j) {
+        const int n = n0 + (wn * WN + j) * 32 + li;
         float *ce = (g.c_up && (n & 32) ? g.c_up : g.c) + (size_t)e * g.c_e;
         const int col = g.c_up ? 32 * (n >> 6) + (n & 31) : n;
 #pragma unroll
-        for (int i = 0; i < BM; ++i)
+        for (int i = 0; i < WM; ++i)
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
-                const int m = m0 + wm * 32 * BM + 32 * i + 8 * (q >> 2) + 4 * lh + (q & 3);
+                const int m = m0 + (wm * WM + i) * 32 + 8 * (q >> 2) + 4 * lh + (q & 3);
                 float *cp = ce + (size_t)m * g.ldc + col;
                 *cp = g.accumulate ? *cp + acc[i][j][q] : acc[i][j][q];
             }
@@ -987,17 +1027,19 @@ hipError_t launch_moe_backward(const BackwardArgs &b, hipStream_t s) {
             // The widest tile that still gives every CU a workgroup.
             const long cus = device_cus();
             auto tiles = [&](int wm, int wn) { return (long)(M / (64 * wm)) * (N / (64 * wn)) * E; };
-            // The wider tiles run 8 waves (two per SIMD): 128 x 128 as 64 x 32
-            // blocks 4 % faster than 4 waves of 64 x 64, 128 x 64 as 32 x 32
-            // blocks 8 % faster than 4 waves of 64 x 32.
+            // perm / k = the high word of perm * ceil(2^32 / k) (perm k < 2^32:
+            // perm < T k <= 2^31 / 64 and k <= 16), or perm itself for k = 1.
+            const unsigned magic = k > 1 ? (unsigned)((((unsigned long long)1 << 32) + k - 1) / k) : 0;
+            const unsigned one = k > 1 ? 0u : ~0u;
             auto go = [&](auto wm, auto wn) {
                 constexpr int WM = decltype(wm)::value, WN = decltype(wn)::value;
-                constexpr int NWM = WM == 2 && WN == 1 ? 4 : 2;
-                constexpr int NWN = WN == 2 ? 4 : 2;
-                hipLaunchKernelGGL((reduce_mfma_kernel<decltype(gather)::value, WM, WN, NWM, NWN>),
-                                   dim3((unsigned)(N / (64 * WN)), (unsigned)(M / (64 * WM)),
-                                        (unsigned)E),
-                                   dim3(64 * NWM * NWN), 0, s, g);
+                const dim3 grid((unsigned)(N / (64 * WN)), (unsigned)(M / (64 * WM)), (unsigned)E);
+                if (tiles(WM, WN) < 2 * cus)
+                    hipLaunchKernelGGL((reduce_split_kernel<decltype(gather)::value, WM, WN, 2>),
+                                       grid, dim3(512), 0, s, g, magic, one);
+                else
+                    hipLaunchKernelGGL((reduce_split_kernel<decltype(gather)::value, WM, WN, 1>),
+                                       grid, dim3(256), 0, s, g, magic, one);
             };
             using I1 = std::integral_constant<int, 1>;
             using I2 = std::integral_constant<int, 2>;

@@ -234,14 +234,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a, char *smem, int mtg
 #undef MOE_TILE_ROWS
 }
 
-// The split tail of a gate/up launch: whole tiles [0, dp), whole rounds of
-// two workgroups per CU (2 tail_groups); r tiles left over (dp .. dp + r - 1),
-// each in s pieces, one piece per CU at most; r = s = 0 when the tail is not
-// split.
+// The split tail of a gate/up launch: whole tiles [0, dp), a multiple of the
+// CUs (tail_groups); r tiles left over (dp .. dp + r - 1), each in s pieces,
+// one piece per CU at most; r = s = 0 when the tail is not split.
 struct TailLayout { int dp, r, s; };
 __device__ __forceinline__ TailLayout tail_layout(const GemmArgs &a, int ntiles, int nks) {
     const int live = a.tile_off[a.E] * ntiles;
-    const int r = live % (2 * a.tail_groups);
+    const int r = live % a.tail_groups;
     const int sp = r ? min(min(nks, 4), a.tail_groups / r) : 0;
     if (sp < 2) return TailLayout{live, 0, 0};
     return TailLayout{live - r, r, sp};
