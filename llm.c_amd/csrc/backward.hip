@@ -697,7 +697,7 @@ struct SlotRows {
     const int *pieces = nullptr;
     int pcols = 0;
     __device__ int count(int a, int d, int c) const {
-        return pieces ? pieces[(size_t)a * (d / pcols) + c / pcols] : ns;
+        return pieces ? pieces[(size_t)a * ((d + pcols - 1) / pcols) + c / pcols] : ns;
     }
     // The partials of (row, column c) added in order; the first 8 are
     // loaded together (clamped, masked), so none waits for another.

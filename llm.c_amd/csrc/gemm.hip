@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
                 w[kb] = a.gw[slot];
                 yp[kb] = a.ys + slot * a.d + 4 * c;
                 np[kb] = !PARTS ? 1
-                         : a.pieces ? a.pieces[slot * (a.d / a.pieces_cols) + 4 * c / a.pieces_cols]
+                         : a.pieces ? a.pieces[slot * ((a.d + a.pieces_cols - 1) / a.pieces_cols) + 4 * c / a.pieces_cols]
                                     : a.ksplit;
                 np[kb] = max(np[kb], 1);
 #pragma unroll
@@ -327,7 +327,7 @@ hipError_t launch_short_first_order(const int *offsets, const int *tile_off, int
 }
 
 hipError_t launch_combine(const CombineArgs &a, hipStream_t s) {
-    if (a.pieces && (a.pieces_cols <= 0 || a.pieces_cols % 4 || a.d % a.pieces_cols))
+    if (a.pieces && (a.pieces_cols <= 0 || a.pieces_cols % 4))
         return hipErrorInvalidValue;
     if (!a.pieces && a.T <= 8 && a.ksplit > 8 && a.ksplit <= 128) {
         // A few tokens: two partials per lane, up to 64 lanes per output.

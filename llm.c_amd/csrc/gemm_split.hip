@@ -31,8 +31,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a, char *smem, int mtg
     constexpr int MB = 4 / WM;   // 32-row blocks per wave
     // Steps that operands are loaded ahead: one where the sums (128 registers
     // with MB = 4) leave no more, else two (a step is half as long there; the
-    // layers of T = 256, d = 512, F = 2048, E = 16, 32 rows per expert and one
-    // tile per CU, 95 -> 86 us).
+    // layers of T = 256, d = 512, F = 2048, E = 16, 32 rows per expert
+    // and one tile per CU, 95 -> 86 us).
     constexpr int D = MB == 4 ? 1 : 2;
     constexpr int PLANE = kStageBytes / 3, STAGE = kStageBytes;
     const int e = a.tile_expert[mtg];
@@ -51,7 +51,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a, char *smem, int mtg
 
     if (MODE == 1 && npieces > 0)
         for (int r = tid; r < rows; r += kThreads)
-            a.pieces[(size_t)a.perm[row0 + r] * (a.N / BN) + nt] = npieces;
+            a.pieces[(size_t)a.perm[row0 + r] * ((a.N + BN - 1) / BN) + nt] = npieces;
 
     auto src_row = [&](int r) -> size_t {   // (rows past the last reuse it)
         const int p = row0 + min(r, rows - 1);
@@ -344,8 +344,7 @@ hipError_t launch_mode(const GemmArgs &a, hipStream_t s) {
     const GemmPlan pl = gemm_plan(a.N, a.K, a.max_mtiles, MODE == 1);
     if (a.K % KT || a.N % 64) return hipErrorInvalidValue;
     if (MODE == 1 && a.streamk) {
-        if (!a.pieces || a.sk_groups <= 0 || a.sk_bn <= 0 || a.N % a.sk_bn) return hipErrorInvalidValue;
-        if (a.sk_bn == 256) return launch_grouped<MODE, 1, 4>(a, s);
+        if (!a.pieces || a.sk_groups <= 0) return hipErrorInvalidValue;
         if (a.sk_bn == 128) return launch_grouped<MODE, 2, 2>(a, s);
         return hipErrorInvalidValue;
     }
@@ -454,10 +453,11 @@ int device_cus() {
 
 GemmPlan gemm_plan(int N, int K, int max_mtiles, bool allow_split) {
     GemmPlan p{0, 1};
-    if (N % 256 == 0) p.bn = 256;
-    else if (N % 128 == 0) p.bn = 128;
-    else if (N % 64 == 0) p.bn = 64;
-    else return p;
+    // A last tile may reach past N: its waves without columns only help
+    // staging A, so wide tiles lose nothing while they are few.  (T = 1003,
+    // d = 320, F = 1376, E = 12, top-3: 108.5 us, with 64-column tiles 133.)
+    if (N % 64) return p;
+    p.bn = N % 256 == 0 || N >= 1024 ? 256 : N > 64 ? 128 : 64;
     if (allow_split) {
         // Down projection: the widest tile, and the reduction split (its
         // partials are added by the combine) until the workgroups cover the
@@ -466,7 +466,7 @@ GemmPlan gemm_plan(int N, int K, int max_mtiles, bool allow_split) {
         // slices) unless the grid is tiny.  Measured at T=4096, d=512,
         // F=2048, E=8: no split 0.568 ms per layer, 2 splits 0.489, 4 0.501.
         const long slots = (long)device_cus() * (p.bn == 256 ? 1 : p.bn == 128 ? 2 : 3);
-        const long blocks = (long)max_mtiles * (N / p.bn);
+        const long blocks = (long)max_mtiles * ((N + p.bn - 1) / p.bn);
         const int min_k = blocks * 4 < slots ? 128 : 512;
         while (p.ksplit < 4 && blocks * p.ksplit < slots && K % (2 * p.ksplit * KT) == 0 &&
                K / (2 * p.ksplit) >= min_k)
@@ -478,9 +478,9 @@ GemmPlan gemm_plan(int N, int K, int max_mtiles, bool allow_split) {
     // across more waves, so they shrink only to 128 columns, and only tiny
     // grids go to 64.
     constexpr size_t kTarget = 1024;
-    auto waves = [&](int bn) { return (size_t)max_mtiles * (N / bn) * (bn / 32); };
+    auto waves = [&](int bn) { return (size_t)max_mtiles * ((N + bn - 1) / bn) * (bn / 32); };
     while (p.bn > 128 && waves(p.bn) < kTarget) p.bn /= 2;
-    if (p.bn > 64 && waves(p.bn) < kTarget / 4 && N % 64 == 0) p.bn = 64;
+    if (p.bn > 64 && waves(p.bn) < kTarget / 4) p.bn = 64;
     return p;
 }
 
@@ -488,16 +488,16 @@ constexpr int kSkBN = 128, kSkPerCu = 2;
 DownPlan down_plan(int N, int K, int max_mtiles, size_t n) {
     const GemmPlan g = gemm_plan(N, K, max_mtiles, true);
     DownPlan p{g.bn, g.ksplit, 0, 0};
-    if (g.bn < 128 || N % kSkBN || K % KT) return p;
+    if (g.bn < 128 || K % KT) return p;
     // Stream-K when the tiles make fewer than ~4 rounds of two workgroups per
     // CU: every workgroup gets the same number of K slices, where whole tiles
     // (or tiles split a fixed 2 or 4 ways) leave a partial last round.
     const long cus = device_cus();
-    if ((long)max_mtiles * (N / 256) >= 8 * cus) return p;
+    if ((long)max_mtiles * ((N + 255) / 256) >= 8 * cus) return p;
     const long nks = K / KT;
     // The fewest live tiles n rows can make (all rows in full m-tiles) set
     // the shortest run per workgroup, hence the most pieces a tile can have.
-    const long tiles_min = (long)((n + BM - 1) / BM) * (N / kSkBN);
+    const long tiles_min = (long)((n + BM - 1) / BM) * ((N + kSkBN - 1) / kSkBN);
     const long units_min = tiles_min * nks;
     // At least 4 slices per workgroup on small problems.
     const long groups = std::max(1L, std::min(kSkPerCu * cus, units_min / 4));
@@ -512,7 +512,7 @@ DownPlan down_plan(int N, int K, int max_mtiles, size_t n) {
 int gateup_tail_groups(int N, int K, int max_mtiles) {
     const GemmPlan g = gemm_plan(N, K, max_mtiles, false);
     const long cus = device_cus();
-    if (g.bn != 256 || K % KT || K / KT < 2 || (long)max_mtiles * (N / 256) >= 8 * cus) return 0;
+    if (g.bn != 256 || N % 256 || K % KT || K / KT < 2 || (long)max_mtiles * (N / 256) >= 8 * cus) return 0;
     return (int)cus;
 }
 

@@ -1240,7 +1240,7 @@ struct FwdPlan {
     int streamk = 0, sk_groups = 0, sk_bn = 0;   // down projection in stream-K form (moe::down_plan)
     size_t h_floats = 0;    // H [n x F] (grouped GEMMs, unfused decode)
     size_t ys_floats = 0;   // per-slot products / split-K partials
-    size_t pieces_ints = 0; // stream-K piece counts [n][d / sk_bn]
+    size_t pieces_ints = 0; // stream-K piece counts [n][ceil(d / sk_bn)]
     int gu_tail = 0;        // gate/up split tail: workgroups per round (moe::gateup_tail_groups)
     size_t gu_part_floats = 0;  // its pieces
     size_t order_ints = 0;  // the down projection's short-first m-tile order (whole tiles, >= 4 rounds)
@@ -1254,7 +1254,7 @@ struct FwdBufs {
     int *counts = nullptr, *offsets = nullptr, *tile_off = nullptr, *tile_expert = nullptr;
     int *perm = nullptr;    // [n]
     float *h = nullptr, *ys = nullptr;
-    int *pieces = nullptr;     // [n][d / sk_bn] (stream-K down projection)
+    int *pieces = nullptr;     // [n][ceil(d / sk_bn)] (stream-K down projection)
     float *gu_part = nullptr;  // gate/up split-tail pieces
     int *order = nullptr;      // [max_mtiles] m-tile order of the down projection
     int *counters = nullptr;   // kMaxCounters ints, zero between launches
@@ -1313,7 +1313,7 @@ int plan_forward(const MoeHipLayer *L, int T, FwdPlan *p, bool probs_given) {
         p->streamk = dp.streamk;
         p->sk_groups = dp.groups;
         p->sk_bn = dp.bn;
-        p->pieces_ints = dp.streamk ? n * (size_t)(d / dp.bn) : 0;
+        p->pieces_ints = dp.streamk ? n * (size_t)((d + dp.bn - 1) / dp.bn) : 0;
         p->gu_tail = moe::gateup_tail_groups(2 * F, d, p->max_mtiles);
         p->gu_part_floats = (size_t)p->gu_tail * moe::kGemmBM * 256;
         if (!dp.streamk && dp.slots == 1 && dp.bn == 256 &&
@@ -1722,7 +1722,7 @@ int moe_hip_backward_dev(MoeHipLayer *L, const float *x, int T, const float *dou
     // dgw, inv [n]; dlogits [T x E].
     const size_t nF = n * F, nd = n * d, ndh = moe::backward_dh_floats(n, d, F, E);
     const size_t ysplits = (size_t)moe::backward_slot_splits(d, F, max_mtiles, n);
-    const size_t npieces = engine && d % 128 == 0 ? n * (size_t)(d / 128) : 0;
+    const size_t npieces = engine ? n * (size_t)((d + 127) / 128) : 0;
     const size_t ntail = moe::backward_tail_floats(d, F, max_mtiles);
     // (the split-tail pieces last, 256-byte aligned)
     const size_t tail_off = (3 * nF + ndh + (ysplits + 1) * nd + 2 * n + (size_t)T * E + npieces +

@@ -108,7 +108,7 @@ struct CombineArgs {
     int ksplit;          // partial products per slot (1 for the GEMM path)
     size_t split_stride; // floats between consecutive partials
     // With pieces: slot a's columns [pieces_cols j, pieces_cols (j + 1)) add
-    // pieces[a * (d / pieces_cols) + j] partials instead of ksplit.
+    // pieces[a * ceil(d / pieces_cols) + j] partials instead of ksplit.
     const int *pieces = nullptr;
     int pieces_cols = 0;
 };
@@ -261,7 +261,7 @@ struct BackwardArgs {
     float aux_coef;
     float *G, *U, *H, *dH, *Y, *dY, *dgw, *dlogits;
     int *inv;
-    int *pieces = nullptr;   // [n][d / 128] when a down_plan is stream-K
+    int *pieces = nullptr;   // [n][ceil(d / 128)] when a down_plan is stream-K
     // Split-tail pieces of the GU recompute and dH products (engine path),
     // backward_tail_floats(...) floats, or null for whole tiles only.
     float *tail_part = nullptr;
