@@ -898,9 +898,10 @@ size_t backward_dh_floats(size_t n, int d, int F, int E) {
     return std::max(n * (size_t)F, (size_t)d * E + E);
 }
 
-size_t backward_tail_floats(int d, int F, int max_mtiles) {
+size_t backward_tail_floats(int d, int F, int max_mtiles, int E) {
     if (!backward_engine_ok(d, F)) return 0;
-    const int g = std::max(gateup_tail_groups(2 * F, d, max_mtiles), gateup_tail_groups(F, d, max_mtiles));
+    const int g = std::max(gateup_tail_groups(2 * F, d, max_mtiles, E),
+                           gateup_tail_groups(F, d, max_mtiles, E));
     return (size_t)g * kGemmBM * 256;
 }
 
@@ -945,7 +946,7 @@ hipError_t launch_moe_backward(const BackwardArgs &b, hipStream_t s) {
         gu.a = b.x; gu.b = b.wgu; gu.c = GU; gu.K = d; gu.N = 2 * F; gu.ldc = 2 * F;
         gu.c2 = b.H; gu.ldc2 = F;
         if (b.tail_part) {
-            gu.tail_groups = gateup_tail_groups(2 * F, d, b.max_mtiles);
+            gu.tail_groups = gateup_tail_groups(2 * F, d, b.max_mtiles, E);
             gu.tail_part = b.tail_part;
         }
         BWD_TRY(launch_gemm_bwd(gu, 2, s));
@@ -966,7 +967,7 @@ hipError_t launch_moe_backward(const BackwardArgs &b, hipStream_t s) {
         GemmArgs gh = g;
         gh.a = b.dY; gh.b = b.wdTT; gh.c = GU; gh.K = d; gh.N = F; gh.ldc = 2 * F;
         if (b.tail_part) {
-            gh.tail_groups = gateup_tail_groups(F, d, b.max_mtiles);
+            gh.tail_groups = gateup_tail_groups(F, d, b.max_mtiles, E);
             gh.tail_part = b.tail_part;
         }
         BWD_TRY(launch_gemm_bwd(gh, 3, s));

@@ -348,7 +348,7 @@ hipError_t launch_mode(const GemmArgs &a, hipStream_t s) {
         if (a.sk_bn == 128) return launch_grouped<MODE, 2, 2>(a, s);
         return hipErrorInvalidValue;
     }
-    if (a.ksplit != (MODE == 1 ? pl.ksplit : 1)) return hipErrorInvalidValue;
+    if (a.ksplit < 1 || (a.K / KT) % a.ksplit || (MODE != 1 && a.ksplit != 1)) return hipErrorInvalidValue;
     if (MODE != 1 && a.tail_groups > 0 && (!a.tail_part || a.N % 256 || pl.bn != 256))
         return hipErrorInvalidValue;
     switch (pl.bn) {
@@ -509,9 +509,15 @@ DownPlan down_plan(int N, int K, int max_mtiles, size_t n) {
     return p;
 }
 
-int gateup_tail_groups(int N, int K, int max_mtiles) {
+int gateup_tail_groups(int N, int K, int max_mtiles, int E) {
     const GemmPlan g = gemm_plan(N, K, max_mtiles, false);
     const long cus = device_cus();
+    // Less than one round of whole tiles is not split: the pieces' sums and
+    // their own launch cost more than the CUs they fill (T = 512, d = 512, F =
+    // 2048, E = 8 through the host drop-in 285 us split, 262 whole; 256 tiles
+    // or more: the backward of T = 4096, d = 256, F = 1024 419 against 423).
+    const long min_tiles = (long)(max_mtiles - E) * (N / 256);
+    if (min_tiles < cus) return 0;
     if (g.bn != 256 || N % 256 || K % KT || K / KT < 2 || (long)max_mtiles * (N / 256) >= 8 * cus) return 0;
     return (int)cus;
 }

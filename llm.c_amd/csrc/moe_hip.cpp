@@ -1263,7 +1263,9 @@ struct FwdBufs {
 
 // probs_given: the caller takes the router probabilities (the general
 // routing kernels then need no logits buffer of their own).
-int plan_forward(const MoeHipLayer *L, int T, FwdPlan *p, bool probs_given) {
+// lean: 1 without the gate/up split tail, 2 without split sums at all.
+int plan_level(const MoeHipLayer *L, int T, FwdPlan *p, bool probs_given, int lean) {
+    *p = FwdPlan{};
     const int d = L->d, F = L->F, E = L->E, k = L->k;
     const size_t n = (size_t)T * k;
     if (n > (size_t)0x7fffffff / (size_t)(F > d ? F : d))
@@ -1308,13 +1310,14 @@ int plan_forward(const MoeHipLayer *L, int T, FwdPlan *p, bool probs_given) {
     } else {
         // Small grids split the down projection's reduction (a fixed split,
         // or stream-K pieces); the combine adds the partials in order.
-        const moe::DownPlan dp = moe::down_plan(d, F, p->max_mtiles, n);
+        moe::DownPlan dp = moe::down_plan(d, F, p->max_mtiles, n);
+        if (lean >= 2) dp = moe::DownPlan{dp.bn, 1, 0, 0};
         p->ksplit = dp.slots;
         p->streamk = dp.streamk;
         p->sk_groups = dp.groups;
         p->sk_bn = dp.bn;
         p->pieces_ints = dp.streamk ? n * (size_t)((d + dp.bn - 1) / dp.bn) : 0;
-        p->gu_tail = moe::gateup_tail_groups(2 * F, d, p->max_mtiles);
+        p->gu_tail = lean ? 0 : moe::gateup_tail_groups(2 * F, d, p->max_mtiles, E);
         p->gu_part_floats = (size_t)p->gu_tail * moe::kGemmBM * 256;
         if (!dp.streamk && dp.slots == 1 && dp.bn == 256 &&
             (long)p->max_mtiles * (d / 256) >= 8L * moe::device_cus())
@@ -1384,6 +1387,20 @@ void carve_bufs(const MoeHipLayer *L, const FwdPlan &p, char *base, size_t cap, 
     c.wide.ints = p.wide_ints ? static_cast<int *>(take(sizeof(int) * p.wide_ints)) : nullptr;
     *need = off;
     if (off <= cap) *b = c;
+}
+
+// A forward whose temporaries fit the allocation-free entry point's scratch
+// in a leaner form only takes that form, in every entry point (so that all
+// give the same bits); one that does not fit in any form takes the full one.
+int plan_forward(const MoeHipLayer *L, int T, FwdPlan *p, bool probs_given) {
+    for (int lean = 0; lean < 3; ++lean) {
+        TRY(plan_level(L, T, p, probs_given, lean));
+        FwdBufs b;
+        size_t need = 0;
+        carve_bufs(L, *p, nullptr, 0, &b, &need);
+        if (need <= kScratchBytes) return MOE_HIP_OK;
+    }
+    return plan_level(L, T, p, probs_given, 0);
 }
 
 }  // namespace
@@ -1723,7 +1740,7 @@ int moe_hip_backward_dev(MoeHipLayer *L, const float *x, int T, const float *dou
     const size_t nF = n * F, nd = n * d, ndh = moe::backward_dh_floats(n, d, F, E);
     const size_t ysplits = (size_t)moe::backward_slot_splits(d, F, max_mtiles, n);
     const size_t npieces = engine ? n * (size_t)((d + 127) / 128) : 0;
-    const size_t ntail = moe::backward_tail_floats(d, F, max_mtiles);
+    const size_t ntail = moe::backward_tail_floats(d, F, max_mtiles, E);
     // (the split-tail pieces last, 256-byte aligned)
     const size_t tail_off = (3 * nF + ndh + (ysplits + 1) * nd + 2 * n + (size_t)T * E + npieces +
                              63) & ~(size_t)63;

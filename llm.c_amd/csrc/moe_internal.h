@@ -275,7 +275,7 @@ bool backward_engine_ok(int d, int F);
 // n = T * k.
 int backward_slot_splits(int d, int F, int max_mtiles, size_t n);
 // Floats of BackwardArgs::tail_part the engine path uses (0: none).
-size_t backward_tail_floats(int d, int F, int max_mtiles);
+size_t backward_tail_floats(int d, int F, int max_mtiles, int E);
 // Floats of BackwardArgs::dH: n x F, and at least one row chunk of the
 // router gradient's partials (d E + E), which reuse it at the end.
 size_t backward_dh_floats(size_t n, int d, int F, int E);
@@ -320,7 +320,7 @@ DownPlan down_plan(int N, int K, int max_mtiles, size_t n);
 // 0 for whole tiles only: used when 256-column tiles make fewer than 4
 // rounds, where the last, partial round is a large share of the launch.
 // The pieces take at most kGemmBM * 256 * groups floats.
-int gateup_tail_groups(int N, int K, int max_mtiles);
+int gateup_tail_groups(int N, int K, int max_mtiles, int E);
 
 // Compute units of the current device (cached; 256 on MI355X).
 int device_cus();

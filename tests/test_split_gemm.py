@@ -85,3 +85,19 @@ def test_limits(T, d, F, where, value):
     # (3e-6 of the norm, as above; one output may cancel terms of the large
     # feature, so single elements have no relative bound)
     assert orc.rel_l2(out[fin], ref[fin]) < 3e-6
+
+
+# Layers whose temporaries fit the allocation-free entry point's scratch only
+# without the split tail, and only without split sums.
+@pytest.mark.parametrize("T,d,F,E,k", [(4096, 512, 2048, 8, 2), (6000, 320, 1376, 12, 3), (1003, 320, 1376, 12, 3)])
+def test_same_plan_without_allocation(T, d, F, E, k):
+    mh.set_expert_path(0)
+    layer = mh.Layer(d, F, E, k)
+    layer.fill_synthetic(5, 0.02, 0.02)
+    x, a, b = (mh.DeviceArray((T, d)) for _ in range(3))
+    mh.fill_normal_dev(x.ptr, T * d, 5, 0, 0.0, 1.0)
+    layer.forward_dev(x.ptr, T, a.ptr)
+    layer.forward_dev_noalloc(x.ptr, T, b.ptr)
+    mh.synchronize()
+    assert np.array_equal(a.to_host().view(np.uint32), b.to_host().view(np.uint32))
+    layer.close()
