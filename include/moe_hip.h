@@ -366,8 +366,8 @@ int moe_hip_eval_exp(int which, const float *x, float *y, size_t n, void *stream
 
 /* Calibration hook for hardware memory counters (no counterpart in the
  * reference): reads `bytes` of device memory at src (a nonzero multiple of
- * 32 MiB) through one load path of the kernels, mode 0 = global-to-LDS DMA
- * (the grouped GEMMs' operand loads), 1 = vector loads, 2 = non-temporal
+ * 32 MiB) through one load path, mode 0 = global-to-LDS DMA (the decode
+ * kernels' rows), 1 = vector loads (the grouped GEMMs' operands), 2 = non-temporal
  * vector loads (the decode weight stream), and writes 1024 per-workgroup
  * sums to out. */
 int moe_hip_read_probe(const void *src, size_t bytes, int mode, float *out, void *stream);

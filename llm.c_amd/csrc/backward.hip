@@ -17,9 +17,10 @@
 //              E f / T; dlogits = p (dp - <dp, p>); dW_r = X^T dlogits
 //   dx         = sum over the token's slots of dXr + dlogits W_r^T
 //
-// Two fp32 tiled GEMMs do the products: rows_gemm over the dispatch tile
-// schedule (one expert per 128-row tile), reduce_gemm with the reduction
-// over an expert's rows.  Every sum runs in a fixed order (deterministic).
+// The row products run on the forward's grouped GEMMs (gemm_split.hip), the
+// weight gradients on reduce_split_kernel (the reduction over an expert's
+// rows); shapes they do not tile on the fp32 rows_mfma, rows_gemm and
+// reduce_gemm kernels.  Every sum runs in a fixed order (deterministic).
 #include "gemm_split.h"
 #include "moe_internal.h"
 #include "moe_math.h"
@@ -281,7 +282,7 @@ struct ReduceGemm {
     int ldc;
     const int *offsets;
     int nrows, chunk, M, N, accumulate, vec_a, vec_b;
-    // reduce_mfma_kernel only: N runs over [G | U]'s 2F packed columns and
+    // reduce_split_kernel only: N runs over [G | U]'s 2F packed columns and
     // column n's product goes to c (gate, n % 64 < 32) or c_up (up) at
     // feature 32 (n / 64) + n % 32.
     float *c_up = nullptr;
@@ -689,7 +690,7 @@ __global__ __launch_bounds__(256) void swiglu_bwd_kernel(float *G, float *U, con
 // Where an expert GEMM left its [T k x d] rows: by dispatch position, or by
 // slot as ns partials ys apart (summed in order).
 // With pieces (a stream-K GEMM): slot a's columns [pcols j, pcols (j + 1))
-// hold pieces[a * (d / pcols) + j] partials instead of ns.
+// hold pieces[a * ceil(d / pcols) + j] partials instead of ns.
 struct SlotRows {
     const float *p;
     int by_slot, ns;

@@ -1,5 +1,5 @@
-// gemm.hip — grouped expert GEMMs on the fp32 matrix cores of gfx950, plus
-// the combine, weight packing and synthetic fill kernels.
+// gemm.hip — the combine, weight packing, m-tile order, synthetic fill and copy
+// kernels around the grouped expert GEMMs (gemm_split.hip).
 //
 // Layout (device, packed once at upload), per expert a matrix of N packed
 // rows by K, stored as 16 x 16 tiles ("units", 1 KB) in MFMA operand order:
@@ -11,36 +11,6 @@
 //   gate/up  wgu [E][2F rows][d]: packed rows 64*fb + c hold gate feature
 //            32*fb + c (c < 32) and up feature 32*fb + c - 32 (c >= 32).
 //   down     wdT [E][d rows][F]: row n holds W_down[:, n].
-// The rows of one expert's m-tile are consecutive dispatch positions
-// offsets[e] + m; gate/up gathers them straight from x through perm.
-//
-// Work decomposition: the grid enumerates (m-tile, n-tile) pairs over the
-// flat per-expert m-tile list built by the dispatch kernel (tile_off), so a
-// hot expert simply owns more tiles; blocks past the live tile count exit.
-//
-// Each workgroup computes a 128 x (64*WN) tile with 2 x WN waves of 64 x 64.
-// A wave issues v_mfma_f32_32x32x2f32 on 2 x 2 sub-tiles.  K is staged
-// through LDS in 32-wide slices (three buffers for 256-column tiles, two for
-// narrower ones); a lane of half h (lane/32) feeds the MFMA's k-row h with
-// the slice's elements 16h..16h+15 in turn, so both operands come from LDS
-// as 128-bit reads.
-// Both operands go global -> LDS by DMA (global_load_lds_dwordx4, one wave
-// instruction = 64 lanes x 16 bytes into 1 KB of LDS), one or two slices
-// ahead of the MFMAs: no registers or LDS store instructions carry the tiles.
-//   B  the packed 1 KB units are copied whole (unit layout in LDS);
-//   A  a unit is 8 whole gathered rows (128 B each, full cache lines), each
-//      row's eight 16-byte chunks permuted by XOR with row % 8 so the
-//      fragment reads are free of bank conflicts.
-// Measured on the gate/up GEMM of the large layer (ms): register staging
-// with the fill in one burst 35.3, spread over the slice 34.5, B by DMA 33.8,
-// both by DMA 33.1.  The DMA is waited for explicitly (vmcnt) before the
-// barrier that ends the slice: s_barrier orders LDS accesses, not loads in
-// flight.
-// Fragments: a wave reads the slice's four quarter-steps into four register
-// sets, set q + 1 while set q's MFMAs run; the last quarter's MFMAs run
-// after the barrier, under the next slice's first reads.  A register that an
-// MFMA still in the pipe reads is never written meanwhile (such a write
-// waits for that MFMA to complete, draining the pipe): 33.0 -> 32.6 ms.
 #include "moe_internal.h"
 #include "moe_math.h"
 #include "synth.h"
@@ -51,21 +21,13 @@ namespace moe {
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int BM = kGemmBM;   // 128
-// LDS buffers per operand: three for 256-column tiles (144 KB, one
-// workgroup per CU either way), two for narrower tiles (whose workgroups
-// share a CU).
-constexpr int gemm_stages(int wn) { return wn == 4 ? 3 : 2; }
-
 // One wave instruction of LDS DMA: lane i's 16 bytes at g go to LDS byte
 // address lds + 16 i (lds wave-uniform, passed in M0).  Written as asm: the
 // compiler books its own LDS DMA builtin as an LDS access as well as a
-// vector load, and then waits for every LDS read with lgkmcnt(0) while a DMA
-// is in flight, which would stall each fragment read ahead.  The DMA counts
-// on vmcnt only, and every slice waits for it (GEMM_WAIT_VMCNT) before the
-// barrier after which its LDS is read.
+// vector load.  The DMA counts on vmcnt only and is waited for explicitly
+// (GEMM_WAIT_VMCNT) before the barrier after which its LDS is read.
 __device__ __forceinline__ void gemm_dma16(const float *g, unsigned lds) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(g), "{m0}"(lds) : "memory");
 }
@@ -464,7 +426,7 @@ hipError_t launch_fill_normal(float *dst, size_t n, uint64_t seed, uint64_t stre
 }
 
 // A read of known size through one load path (counter calibration): MODE 0
-// the grouped GEMMs' LDS DMA (global_load_lds_dwordx4), 1 buffer loads into
+// LDS DMA (global_load_lds_dwordx4), 1 buffer loads into
 // registers with the default cache policy, 2 the same loads non-temporal
 // (the decode weight stream).  Workgroup b (4 waves) reads bytes [b span,
 // (b + 1) span) in 4 KB steps, eight 1 KB wave instructions in flight; the

@@ -459,12 +459,11 @@ GemmPlan gemm_plan(int N, int K, int max_mtiles, bool allow_split) {
     if (N % 64) return p;
     p.bn = N % 256 == 0 || N >= 1024 ? 256 : N > 64 ? 128 : 64;
     if (allow_split) {
-        // Down projection: the widest tile, and the reduction split (its
-        // partials are added by the combine) until the workgroups cover the
-        // CUs once: blocks of 256 columns hold a CU each, narrower ones share
-        // it 2 or 3 ways.  A split keeps >= 512 reduction elements (16 LDS
-        // slices) unless the grid is tiny.  Measured at T=4096, d=512,
-        // F=2048, E=8: no split 0.568 ms per layer, 2 splits 0.489, 4 0.501.
+        // Down projection where stream-K is not taken (one 64-column tile,
+        // or several rounds): the widest tile, and for small grids the
+        // reduction split (its partials are added by the combine) until the
+        // workgroups cover the CUs.  A split keeps >= 512 reduction elements
+        // unless the grid is tiny.
         const long slots = (long)device_cus() * (p.bn == 256 ? 1 : p.bn == 128 ? 2 : 3);
         const long blocks = (long)max_mtiles * ((N + p.bn - 1) / p.bn);
         const int min_k = blocks * 4 < slots ? 128 : 512;
@@ -473,17 +472,19 @@ GemmPlan gemm_plan(int N, int K, int max_mtiles, bool allow_split) {
             p.ksplit *= 2;
         return p;
     }
-    // Without a split: waves in flight for tile width bn (bn / 32 waves per
-    // workgroup); aim for ~4 per SIMD.  Wider tiles reuse each loaded tile
-    // across more waves, so they shrink only to 128 columns, and only tiny
-    // grids go to 64.
-    constexpr size_t kTarget = 1024;
-    auto waves = [&](int bn) { return (size_t)max_mtiles * ((N + bn - 1) / bn) * (bn / 32); };
-    while (p.bn > 128 && waves(p.bn) < kTarget) p.bn /= 2;
-    if (p.bn > 64 && waves(p.bn) < kTarget / 4) p.bn = 64;
+    // Without a split: 256-column tiles (each column split once per 128
+    // rows) while they make half a workgroup per CU, 128-column ones (split
+    // by both wave rows) down to 64 workgroups, 64-column ones below.
+    auto tiles = [&](int bn) { return (long)max_mtiles * ((N + bn - 1) / bn); };
+    if (p.bn > 128 && tiles(256) < 128) p.bn = 128;
+    if (p.bn > 64 && tiles(p.bn) * (p.bn / 64) < 128) p.bn = 64;
     return p;
 }
 
+// Stream-K takes 128-column tiles over two workgroups per CU: as many partials
+// per slot as 256-column tiles over one per CU, with twice the waves (T =
+// 4096, d = 256, F = 1024, E = 8: 115.8 us per layer against 121; 256 columns
+// over two per CU 126.5, 128 over four 132).
 constexpr int kSkBN = 128, kSkPerCu = 2;
 DownPlan down_plan(int N, int K, int max_mtiles, size_t n) {
     const GemmPlan g = gemm_plan(N, K, max_mtiles, true);

@@ -305,7 +305,7 @@ hipError_t launch_fill_normal(float *dst, size_t n, uint64_t seed,
                               hipStream_t s);
 
 // Tile width (64, 128 or 256 columns) and reduction split of a grouped GEMM
-// launch, sized for ~1024 waves in flight (gemm.hip).
+// launch (gemm_split.hip).
 struct GemmPlan {
     int bn, ksplit;
 };
@@ -319,8 +319,9 @@ struct DownPlan {
 };
 DownPlan down_plan(int N, int K, int max_mtiles, size_t n);
 // Workgroups per round for a gate/up launch with a split tail (the CUs), or
-// 0 for whole tiles only: used when 256-column tiles make fewer than 4
-// rounds, where the last, partial round is a large share of the launch.
+// 0 for whole tiles only: used when 256-column tiles make between one and
+// eight per CU, where the last, partial round is a large share of the launch.
+// max_mtiles: ceil(n / kGemmBM) + E.
 // The pieces take at most kGemmBM * 256 * groups floats.
 int gateup_tail_groups(int N, int K, int max_mtiles, int E);
 
