@@ -500,8 +500,13 @@ DownPlan down_plan(int N, int K, int max_mtiles, size_t n) {
     // the shortest run per workgroup, hence the most pieces a tile can have.
     const long tiles_min = (long)((n + BM - 1) / BM) * ((N + kSkBN - 1) / kSkBN);
     const long units_min = tiles_min * nks;
-    // At least 4 slices per workgroup on small problems.
-    const long groups = std::max(1L, std::min(kSkPerCu * cus, units_min / 4));
+    // At least 4 slices per workgroup on small problems, counted on the most
+    // tiles the rows can make: few rows over many experts make an m-tile each
+    // (T = 15, d = 192, F = 4768, E = 170, top-7: counted on the fewest, 74
+    // workgroups did the work of 160 tiles).  The partials stay bounded:
+    // slots n N is about groups tiles at most.
+    const long units_max = (long)max_mtiles * ((N + kSkBN - 1) / kSkBN) * nks;
+    const long groups = std::max(1L, std::min(kSkPerCu * cus, units_max / 4));
     const long per_min = (units_min + groups - 1) / groups;
     p.bn = kSkBN;
     p.streamk = 1;
