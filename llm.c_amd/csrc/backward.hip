@@ -518,34 +518,33 @@ __global__ __launch_bounds__(256 * KG, 2) void reduce_split_kernel(ReduceGemm g,
 #pragma unroll
         for (int i = 0; i < WM * WN * 16; ++i) acc[i / (16 * WN)][i / 16 % WN][i % 16] += x[64 * i];
     }
-    // Not all finite: again as float products (gemm_split.h), rows r + lh at
-    // a time.
-    float chk = 0.f;
+    // Sums that are not finite: again as float products (gemm_split.h), rows
+    // r + lh at a time.
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int j = 0; j < WN; ++j)
+        for (int j = 0; j < WN; ++j) {
+            float chk = 0.f;
 #pragma unroll
             for (int q = 0; q < 16; ++q) chk = fmaf(acc[i][j][q], 0.f, chk);
-    if (__ballot(!(chk == 0.f))) {
+            if (!__ballot(!(chk == 0.f))) continue;
+            const float *ca = g.a + m0 + (wm * WM + i) * 32 + li;
+            const float *cb = g.b + n0 + (wn * WN + j) * 32 + li;
+            fx16 f;
 #pragma unroll
-        for (int i = 0; i < WM; ++i)
-#pragma unroll
-            for (int j = 0; j < WN; ++j) {
-                const float *ca = g.a + m0 + (wm * WM + i) * 32 + li;
-                const float *cb = g.b + n0 + (wn * WN + j) * 32 + li;
-#pragma unroll
-                for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
+            for (int q = 0; q < 16; ++q) f[q] = 0.f;
 #pragma unroll 1
-                for (int r = r0; r < r1; r += 2) {
-                    const int row = min(r + lh, r1 - 1);
-                    float x = ca[(GATHER ? token(g.perm[row]) : (size_t)row) * g.lda];
-                    float y = cb[(size_t)row * g.ldb];
-                    if (r + lh >= r1) x = y = 0.f;
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc[i][j], 0, 0, 0);
-                }
+            for (int r = r0; r < r1; r += 2) {
+                const int row = min(r + lh, r1 - 1);
+                float x = ca[(GATHER ? token(g.perm[row]) : (size_t)row) * g.lda];
+                float y = cb[(size_t)row * g.ldb];
+                if (r + lh >= r1) x = y = 0.f;
+                f = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, f, 0, 0, 0);
             }
-    }
+#pragma unroll
+            for (int q = 0; q < 16; ++q)
+                acc[i][j][q] = float_sum_needed(acc[i][j][q]) ? f[q] : acc[i][j][q];
+        }
     // Lane l, register q of a block: row 8 (q / 4) + 4 (l / 32) + q % 4,
     // column l % 32.
 #pragma unroll

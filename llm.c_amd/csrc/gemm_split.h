@@ -26,9 +26,10 @@
 //
 // An infinity or NaN among the operands makes NaNs of the split's remainders
 // where the float sum may be an infinity, and a float above the largest
-// bfloat16 becomes one: a wave whose sums are not all finite computes them
-// again on the fp32 MFMAs, so non-finite results are those of
-// float products.
+// bfloat16 becomes one: sums that are not finite are computed again on the
+// fp32 MFMAs, so non-finite results are those of float products.  The choice
+// is made element by element: no other row's or column's values change an
+// element's bits.
 #pragma once
 #include "moe_internal.h"
 #include "moe_math.h"
@@ -76,6 +77,9 @@ __device__ __forceinline__ fx16 mma(ux4 a, ux4 b, fx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bx8, a),
                                                    __builtin_bit_cast(bx8, b), c, 0, 0, 0);
 }
+
+// A sum of split products to be replaced by the sum of float products.
+__device__ __forceinline__ bool float_sum_needed(float s) { return !(fabsf(s) <= 0x1.fffffep127f); }
 
 // The six term pairs, smallest first.
 constexpr int kPairs = 6;

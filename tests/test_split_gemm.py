@@ -101,3 +101,65 @@ def test_same_plan_without_allocation(T, d, F, E, k):
     mh.synchronize()
     assert np.array_equal(a.to_host().view(np.uint32), b.to_host().view(np.uint32))
     layer.close()
+
+
+def _forward(layer, x):
+    T = len(x)
+    dx, out = mh.DeviceArray.from_host(x), mh.DeviceArray(x.shape)
+    layer.forward_dev(dx.ptr, T, out.ptr)
+    mh.synchronize()
+    return out.to_host()
+
+
+# One expert, so that every row keeps its place.  Gate/up on 64-column tiles,
+# on 256-column ones, and on those with a split tail; down in one tile column
+# and in stream-K form.
+@pytest.mark.parametrize("T,d,F", [(40, 64, 64), (300, 64, 8192), (700, 256, 4096)])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_non_finite_row_leaves_others(T, d, F, value):
+    """A row with a non-finite element: the other rows' bits stay."""
+    layer = mh.Layer(d, F, 1, 1)
+    layer.fill_synthetic(6, 0.05, 0.05)
+    x = orc.synth((T, d), 8, 0, 1.0)
+    ref = _forward(layer, x)
+    bad = [3, T - 1]
+    x[bad, 5] = value
+    out = _forward(layer, x)
+    assert not np.isfinite(out[bad]).any()
+    rest = np.setdiff1d(np.arange(T), bad)
+    assert np.array_equal(out[rest].view(np.uint32), ref[rest].view(np.uint32))
+    layer.close()
+
+
+# The weight gradients' tiles: 64 x 64 and 128 x 64 with two wave groups,
+# 128 x 128 with one (256 rows per expert and more).
+@pytest.mark.parametrize("T,d,F,E", [(200, 64, 64, 2), (1000, 256, 1024, 8), (2048, 512, 2048, 8)])
+def test_non_finite_gradient_leaves_others(T, d, F, E):
+    """An infinity in one element of dout: the infinities that float products
+    make of it in its column of dW_down, and the bits of the other columns and
+    of the other rows' dx stay."""
+    layer = mh.Layer(d, F, E, 1)
+    layer.fill_synthetic(6, 0.05, 0.05)
+    x, dout = orc.synth((T, d), 9, 0, 1.0), orc.synth((T, d), 9, 1, 1.0)
+    dxd, ids = mh.DeviceArray.from_host(x), mh.DeviceArray((T, 1), np.int32)
+    out = mh.DeviceArray((T, d))
+    layer.forward_dev(dxd.ptr, T, out.ptr, None, ids.ptr)
+    res = []
+    for value in (dout[7, 9], np.inf):
+        dout[7, 9] = value
+        outs = [mh.DeviceArray(s) for s in ((T, d), (d, E), (E, d, F), (E, d, F), (E, F, d))]
+        dod = mh.DeviceArray.from_host(dout)
+        layer.backward_dev(dxd.ptr, T, dod.ptr, 0.0, *[a.ptr for a in outs])
+        mh.synchronize()
+        res.append((outs[0].to_host(), outs[4].to_host()))
+    (dx0, dw0), (dx1, dw1) = res
+    e = int(ids.to_host()[7, 0])
+    col = dw1[e][:, 9].copy()
+    wg, wu = layer.get_expert(e)[:2]
+    g, u = (x[7].astype(np.float64) @ w.astype(np.float64) for w in (wg, wu))
+    assert np.array_equal(col, np.sign(g * u) * np.inf)
+    assert not np.isfinite(dx1[7]).any()
+    dw1[e][:, 9], dx1[7] = dw0[e][:, 9], dx0[7]
+    assert np.array_equal(dw0.view(np.uint32), dw1.view(np.uint32))
+    assert np.array_equal(dx0.view(np.uint32), dx1.view(np.uint32))
+    layer.close()
