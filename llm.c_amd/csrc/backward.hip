@@ -518,16 +518,13 @@ __global__ __launch_bounds__(256 * KG, 2) void reduce_split_kernel(ReduceGemm g,
 #pragma unroll
         for (int i = 0; i < WM * WN * 16; ++i) acc[i / (16 * WN)][i / 16 % WN][i % 16] += x[64 * i];
     }
-    // Sums that are not finite: again as float products (gemm_split.h), rows
-    // r + lh at a time.
+    // Sums that are not finite, or too small for the split: again as float
+    // products (gemm_split.h), rows r + lh at a time.
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
-            float chk = 0.f;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) chk = fmaf(acc[i][j][q], 0.f, chk);
-            if (!__ballot(!(chk == 0.f))) continue;
+            if (!any_float_sum(acc[i][j])) continue;
             const float *ca = g.a + m0 + (wm * WM + i) * 32 + li;
             const float *cb = g.b + n0 + (wn * WN + j) * 32 + li;
             fx16 f;

@@ -3,7 +3,8 @@
 //
 // x = h + m + l with h = bf16(x), m = bf16(x - h), l = bf16(x - h - m), each
 // rounded to nearest: 8 + 8 + 8 significant bits hold all 24 of a float, and
-// both subtractions are exact, so the split loses nothing.  A product takes
+// both subtractions are exact, so for 2^-109 <= |x| < 2^128 - 2^119 (and 0)
+// the split loses nothing.  A product takes
 // the six terms down to 2^-16 of the largest (hh, hm, mh, mm, hl, lh); the
 // three left out are below 2^-25 of it, under half an ulp of the float
 // product.  All six go into one float accumulator.  Six
@@ -12,6 +13,8 @@
 // N(0, 0.02) against float64, this against the fp32 MFMA chain: K = 64
 // 1.0e-7 / 1.4e-7, 512 3.4e-7 / 4.0e-7, 2048 7.0e-7 / 7.8e-7, 8192 1.4e-6 /
 // 1.6e-6 (fewer roundings of the running sum: 6 for 16 products, not 16).
+// With only a few nonzero products the terms left out show: four of 64
+// 6.3e-8 / 3.8e-8.
 //
 // Work: 128 x BN tiles (BN = 64 WN) on four waves, WM x WN of (128 / WM) x
 // 64; two such workgroups share a CU, so one's splitting and LDS traffic run
@@ -22,14 +25,21 @@
 //   A  (128 rows, gathered) is split once by the workgroup, each thread 4 k
 //      of 2 rows, and kept in LDS as three planes in MFMA operand order (two
 //      stages of 12 KB, one barrier per step).
-// The loads of the next step are in flight while a step multiplies.
+// The operands of the next step (128- and 64-column tiles: of the next two) are
+// in flight while a step multiplies.
 //
-// An infinity or NaN among the operands makes NaNs of the split's remainders
-// where the float sum may be an infinity, and a float above the largest
-// bfloat16 becomes one: sums that are not finite are computed again on the
-// fp32 MFMAs, so non-finite results are those of float products.  The choice
-// is made element by element: no other row's or column's values change an
-// element's bits.
+// Outside that range the split is not used for the result.  An infinity or
+// NaN among the operands makes NaNs of the remainders where the float sum may
+// be an infinity, and a float above the largest bfloat16 becomes one; under
+// 2^-109 the third term, then the second, falls below bfloat16's smallest
+// subnormal (2^-133).  So a sum that is not finite, or nonzero and below
+// 2^-80, is computed again on the fp32 MFMAs.  The choice is made element by
+// element: no other row's or column's values change an element's bits.  What
+// stays less exact than float products: an operand below 2^-109 that meets one
+// above 2^29 (its sum may pass 2^-80), and one below 2^-134, which counts as
+// zero where a whole sum has no larger ones.  (A layer whose gate sums and H
+// are of the order of 2^-118, d = 256, F = 512: 5.6e-5 from float64 without
+// the rule, below 3e-6 with it.)
 #pragma once
 #include "moe_internal.h"
 #include "moe_math.h"
@@ -79,7 +89,31 @@ __device__ __forceinline__ fx16 mma(ux4 a, ux4 b, fx16 c) {
 }
 
 // A sum of split products to be replaced by the sum of float products.
-__device__ __forceinline__ bool float_sum_needed(float s) { return !(fabsf(s) <= 0x1.fffffep127f); }
+constexpr float kSmallSum = 0x1p-80f;
+__device__ __forceinline__ bool float_sum_needed(float s) {
+    return !(fabsf(s) >= kSmallSum && fabsf(s) <= 0x1.fffffep127f) && s != 0.0f;
+}
+
+// A wave's 16 sums per lane into the cheaper check that finds all of them
+// fit: chk stays 0 while they are finite, lo is the smallest magnitude (zeros
+// included: their exact check follows, and finds nothing to replace).
+struct SumCheck {
+    float chk = 0.0f, lo = 1.0f;
+    __device__ __forceinline__ void add(fx16 a) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            chk = fmaf(a[r], 0.0f, chk);
+            lo = fminf(lo, fabsf(a[r]));
+        }
+    }
+    __device__ __forceinline__ bool fits() const { return !__ballot(!(chk == 0.0f && lo >= kSmallSum)); }
+};
+__device__ __forceinline__ bool any_float_sum(fx16 a) {
+    bool any = false;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) any |= float_sum_needed(a[r]);
+    return __ballot(any) != 0;
+}
 
 // The six term pairs, smallest first.
 constexpr int kPairs = 6;

@@ -169,37 +169,41 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a, char *smem, int mtg
         default: if constexpr (MB >= 4) loop(std::integral_constant<int, 4>{}); break;
     }
 
-    // Sums that are not finite: again as float products (gemm_split.h).
+    // Sums that are not finite, or too small for the split: again as float
+    // products (gemm_split.h).
+    SumCheck check;
 #pragma unroll
     for (int m = 0; m < MB; ++m) {
         if (m >= nmb) break;
-        float chk = 0.0f;
+        check.add(acc[m][0]);
+        check.add(acc[m][1]);
+    }
+    if (!check.fits()) {
 #pragma unroll
-        for (int n = 0; n < 2; ++n)
+        for (int m = 0; m < MB; ++m) {
+            if (m >= nmb || !(any_float_sum(acc[m][0]) || any_float_sum(acc[m][1]))) continue;
+            const float *ax = a.a + src_row((wm * MB + m) * 32 + li) * K + kb + 8 * lh;
+            fx16 f[2];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) chk = fmaf(acc[m][n][r], 0.0f, chk);
-        if (!__ballot(!(chk == 0.0f))) continue;
-        const float *ax = a.a + src_row((wm * MB + m) * 32 + li) * K + kb + 8 * lh;
-        fx16 f[2];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) f[0][r] = f[1][r] = 0.0f;
+            for (int r = 0; r < 16; ++r) f[0][r] = f[1][r] = 0.0f;
 #pragma unroll 1
-        for (int s = 0; s <= last; ++s) {
-            load_b(S0{}, s);
-            const fx4 x0 = *reinterpret_cast<const fx4 *>(ax + 16 * s);
-            const fx4 x1 = *reinterpret_cast<const fx4 *>(ax + 16 * s + 4);
+            for (int s = 0; s <= last; ++s) {
+                load_b(S0{}, s);
+                const fx4 x0 = *reinterpret_cast<const fx4 *>(ax + 16 * s);
+                const fx4 x1 = *reinterpret_cast<const fx4 *>(ax + 16 * s + 4);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float x = j < 4 ? x0[j & 3] : x1[j & 3];
-                f[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, rb[0][j >> 2][j & 3], f[0], 0, 0, 0);
-                f[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, rb[0][2 + (j >> 2)][j & 3], f[1], 0, 0, 0);
+                for (int j = 0; j < 8; ++j) {
+                    const float x = j < 4 ? x0[j & 3] : x1[j & 3];
+                    f[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, rb[0][j >> 2][j & 3], f[0], 0, 0, 0);
+                    f[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, rb[0][2 + (j >> 2)][j & 3], f[1], 0, 0, 0);
+                }
             }
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    acc[m][n][r] = float_sum_needed(acc[m][n][r]) ? f[n][r] : acc[m][n][r];
         }
-#pragma unroll
-        for (int n = 0; n < 2; ++n)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                acc[m][n][r] = float_sum_needed(acc[m][n][r]) ? f[n][r] : acc[m][n][r];
     }
 
     // Accumulator layout of a 32x32 block: lane l, register r holds

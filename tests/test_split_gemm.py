@@ -1,11 +1,17 @@
 """The grouped GEMMs on split operands (gemm_split.h) at the edges of their
 tiles and at the limits of their number range."""
+import os
+import sys
+
 import numpy as np
 import pytest
 
 import moe_hip as mh
 import orc
 from abi_types import HostMoE
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle"))
+import moe_backward as mb  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -162,4 +168,47 @@ def test_non_finite_gradient_leaves_others(T, d, F, E):
     dw1[e][:, 9], dx1[7] = dw0[e][:, 9], dx0[7]
     assert np.array_equal(dw0.view(np.uint32), dw1.view(np.uint32))
     assert np.array_equal(dx0.view(np.uint32), dx1.view(np.uint32))
+    layer.close()
+
+
+# The operands' range goes down to the smallest floats.  Gate sums see only the
+# scaled half of a row, up sums the other half, so H (and the down sums) take
+# the scale once; W_down is raised to bring the outputs back among the normal
+# floats.
+@pytest.mark.parametrize("T,d,F", [(40, 64, 64), (700, 256, 512)])
+@pytest.mark.parametrize("e", [70, 90, 109, 118, 125])
+def test_small_operands(T, d, F, e):
+    hw = _layer(d, F, 2, 1, 11)
+    x = orc.synth((T, d), 6, 0, 1.0)
+    x[:, d // 2:] *= np.float32(2.0 ** -e)
+    hw.wg[:, :d // 2] = 0
+    hw.wu[:, d // 2:] = 0
+    hw.wd *= np.float32(2.0 ** 24)
+    out, probs, ids = mh.moe_forward(x, hw)
+    # (x * 2^-125 has subnormal elements, exact to 2^-149: they enter the
+    # reference as rounded; bound as in test_tile_edges)
+    assert orc.rel_l2(out, _layer64(x, hw, ids, probs)) < 3e-6
+
+
+@pytest.mark.parametrize("e", [90, 115, 118])
+@pytest.mark.parametrize("T,d,F", [(200, 128, 192), (90, 64, 64)])
+def test_small_gradients(T, d, F, e):
+    """Gradients of a loss scaled by 2^-e, to the precision of an unscaled one."""
+    r = np.random.default_rng(T)
+    f = lambda *s: (0.3 * r.standard_normal(s)).astype(np.float32)
+    hw = HostMoE(f(d, 4), f(4, d, F), f(4, d, F), f(4, F, d), 2)
+    x, dout = orc.synth((T, d), 7, 0, 1.0), orc.synth((T, d), 7, 1, 1.0)
+    ids = orc.route(x, hw.wr, 2)[1]
+    g = mb.moe_backward64(x, hw.wr, hw.wg, hw.wu, hw.wd, ids, dout)
+    layer = mh.Layer(d, F, 4, 2)
+    layer.load(hw)
+    outs = dict(dx=mh.DeviceArray((T, d)), dwr=mh.DeviceArray((d, 4)), dwg=mh.DeviceArray((4, d, F)),
+                dwu=mh.DeviceArray((4, d, F)), dwd=mh.DeviceArray((4, F, d)))
+    dxd, dod = mh.DeviceArray.from_host(x), mh.DeviceArray.from_host(dout * np.float32(2.0 ** -e))
+    layer.backward_dev(dxd.ptr, T, dod.ptr, 0.0, *[a.ptr for a in outs.values()])
+    mh.synchronize()
+    for name, a in outs.items():
+        # Chains of up to four sums of at most 192 products each and the
+        # SwiGLU's derivative: under 3e-6 (as above).
+        assert orc.rel_l2(a.to_host().astype(np.float64) * 2.0 ** e, g[name]) < 3e-6, name
     layer.close()
