@@ -1392,14 +1392,23 @@ void carve_bufs(const MoeHipLayer *L, const FwdPlan &p, char *base, size_t cap, 
 // A forward whose temporaries fit the allocation-free entry point's scratch
 // in a leaner form only takes that form, in every entry point (so that all
 // give the same bits); one that does not fit in any form takes the full one.
+// The form is the one that fits without the caller's probs buffer, where one
+// does: asking for the probabilities changes no bits either.
+// What the leaner form costs or gives against the full one, us: d = 512, F =
+// 2048, E = 8, top-2 T = 4096 314 -> 315, 5000 367 -> 383, 6500 471 -> 454; d =
+// 512, F = 1536, E = 16 T = 8000 449 -> 472; d = 1024, F = 512, E = 256, top-8 T =
+// 1700 562 -> 501.  (Between the two, one stream-K workgroup per CU: 364 at T =
+// 5000, but d = 320, F = 1376, E = 12, top-3 T = 5000 282 where no split takes
+// 270.)
 int plan_forward(const MoeHipLayer *L, int T, FwdPlan *p, bool probs_given) {
-    for (int lean = 0; lean < 3; ++lean) {
-        TRY(plan_level(L, T, p, probs_given, lean));
-        FwdBufs b;
-        size_t need = 0;
-        carve_bufs(L, *p, nullptr, 0, &b, &need);
-        if (need <= kScratchBytes) return MOE_HIP_OK;
-    }
+    for (int probs = 0; probs < (is_wide(L->E, L->k) ? 2 : 1); ++probs)
+        for (int lean = 0; lean < 3; ++lean) {
+            TRY(plan_level(L, T, p, probs != 0, lean));
+            FwdBufs b;
+            size_t need = 0;
+            carve_bufs(L, *p, nullptr, 0, &b, &need);
+            if (need <= kScratchBytes) return plan_level(L, T, p, probs_given, lean);
+        }
     return plan_level(L, T, p, probs_given, 0);
 }
 

@@ -109,6 +109,23 @@ def test_same_plan_without_allocation(T, d, F, E, k):
     layer.close()
 
 
+# 300 experts: the general routing kernels, whose logits take 12 MB when the
+# caller has no probs buffer; around 134 MB in all, with and without them.
+@pytest.mark.parametrize("T", [9000, 9600, 10000, 10400])
+def test_same_plan_without_probs(T):
+    mh.set_expert_path(0)
+    d, F, E, k = 512, 512, 300, 2
+    layer = mh.Layer(d, F, E, k)
+    layer.fill_synthetic(5, 0.02, 0.02)
+    x, a, b, probs = (mh.DeviceArray(s) for s in ((T, d), (T, d), (T, d), (T, E)))
+    mh.fill_normal_dev(x.ptr, T * d, 5, 0, 0.0, 1.0)
+    layer.forward_dev(x.ptr, T, a.ptr)
+    layer.forward_dev(x.ptr, T, b.ptr, probs.ptr)
+    mh.synchronize()
+    assert np.array_equal(a.to_host().view(np.uint32), b.to_host().view(np.uint32))
+    layer.close()
+
+
 def _forward(layer, x):
     T = len(x)
     dx, out = mh.DeviceArray.from_host(x), mh.DeviceArray(x.shape)
