@@ -466,13 +466,13 @@ GemmPlan gemm_plan(int N, int K, int max_mtiles, bool allow_split) {
     if (N % 64) return p;
     p.bn = N % 256 == 0 || N >= 1024 ? 256 : N > 64 ? 128 : 64;
     if (allow_split) {
-        // Down projection where stream-K is not taken (one 64-column tile,
-        // or several rounds): the widest tile, and for small grids the
-        // reduction split (its partials are added by the combine) until the
-        // workgroups cover the CUs.  A split keeps >= 512 reduction elements
-        // unless the grid is tiny.
-        const long slots = (long)device_cus() * (p.bn == 256 ? 1 : p.bn == 128 ? 2 : 3);
-        const long blocks = (long)max_mtiles * ((N + p.bn - 1) / p.bn);
+        // Down projection where stream-K is not taken: wide tiles whole (eight
+        // of them per CU and more, or no room for partials); the one 64-column
+        // tile of N = 64 splits its reduction until the workgroups cover the
+        // CUs (its partials are added by the combine), keeping >= 512
+        // reduction elements unless the grid is tiny.
+        if (p.bn > 64) return p;
+        const long slots = 3L * device_cus(), blocks = max_mtiles;
         const int min_k = blocks * 4 < slots ? 128 : 512;
         while (p.ksplit < 4 && blocks * p.ksplit < slots && K % (2 * p.ksplit * KT) == 0 &&
                K / (2 * p.ksplit) >= min_k)

@@ -1311,7 +1311,7 @@ int plan_level(const MoeHipLayer *L, int T, FwdPlan *p, bool probs_given, int le
         // Small grids split the down projection's reduction (a fixed split,
         // or stream-K pieces); the combine adds the partials in order.
         moe::DownPlan dp = moe::down_plan(d, F, p->max_mtiles, n);
-        if (lean >= 2) dp = moe::DownPlan{dp.bn, 1, 0, 0};
+        if (lean >= 2) dp = moe::DownPlan{moe::gemm_plan(d, F, p->max_mtiles, true).bn, 1, 0, 0};
         p->ksplit = dp.slots;
         p->streamk = dp.streamk;
         p->sk_groups = dp.groups;

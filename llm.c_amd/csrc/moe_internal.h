@@ -157,7 +157,7 @@ hipError_t launch_gemm_down(const GemmArgs &a, hipStream_t s);
 // in expert order, then every other m-tile in m-tile order (one workgroup).
 hipError_t launch_short_first_order(const int *offsets, const int *tile_off, int E, int *order,
                                     hipStream_t s);
-// The backward's tile epilogues (gemm.hip), no reduction split:
+// The backward's tile epilogues (gemm_split.hip), no reduction split:
 //   mode 2  gate/up rows gathered like the forward: c = [G | U] per 32-feature
 //           group in the packed column order (ldc = 2F), c2 = H (ldc2 = F);
 //   mode 3  a = dY rows, b = the unit transpose of wdT (N = F, K = d): the
