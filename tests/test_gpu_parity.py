@@ -508,11 +508,11 @@ def test_decode_tiny_guess_differs(k):
 
 
 def test_down_short_first():
-    """A down projection of at least 4 rounds of 256-column tiles (d 2048,
+    """A down projection of at least eight 256-column tiles per CU (d 2048,
     64 experts, a skewed router bias) runs the experts' short last m-tiles
     first: every token against the oracle, and the routes do give short
     m-tiles (97 rows or fewer) to reorder."""
-    T, d, F, E, k = 2048, 2048, 64, 64, 4
+    T, d, F, E, k = 6144, 2048, 64, 64, 4
     say(f"down short-first: T={T} d={d} F={F} E={E} k={k}")
     layer = mh.Layer(d, F, E, k)
     layer.fill_synthetic(23, 0.02, 0.05)
@@ -535,8 +535,10 @@ def test_down_short_first():
     short = int(((m > 0) & (counts - 128 * (m - 1) <= 96)).sum())
     say(f"down short-first: m-tiles {int(m.sum())}, short {short}")
     # (the library takes the order when its m-tile bound, ceil(T k / 128) + E,
-    # makes at least 4 rounds of 256 workgroups)
-    assert short > 0 and ((T * k + 127) // 128 + E) * (d // 256) >= 4 * 256
+    # makes at least eight tiles for each of 256 CUs, which is where stream-K
+    # ends, and the layer does not fit the 128 MiB scratch)
+    assert short > 0 and ((T * k + 127) // 128 + E) * (d // 256) >= 8 * 256
+    assert 4 * T * k * d > 128 << 20
     assert_close(dout.to_host(), o_ref, "down short-first")
     layer.close()
 
