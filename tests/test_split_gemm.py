@@ -229,3 +229,83 @@ def test_small_gradients(T, d, F, e):
         # SwiGLU's derivative: under 3e-6 (as above).
         assert orc.rel_l2(a.to_host().astype(np.float64) * 2.0 ** e, g[name]) < 3e-6, name
     layer.close()
+
+
+# Widths past 1024 that 256 does not divide: gate/up's last 256-column tile
+# reaches past N (64 features of its 128 here; with 12 experts 96 of 128).
+@pytest.mark.parametrize("T,d,F,E,k", [(700, 64, 5440, 2, 1), (1003, 320, 1376, 12, 3)])
+def test_wide_tiles_past_the_width(T, d, F, E, k):
+    hw = _layer(d, F, E, k, T)
+    x = orc.synth((T, d), 12, 0, 1.0)
+    out, probs, ids = mh.moe_forward(x, hw)
+    # (as in test_tile_edges, the down sums up to 5440 products long)
+    assert orc.rel_l2(out, _layer64(x, hw, ids, probs)) < 4e-6
+
+
+# gate/up on 256-column tiles (one wave for 128 rows, last m-tiles of one to
+# four 32-row blocks), without and with a split tail (2 and 4 pieces).
+@pytest.mark.parametrize("T,d,F", [(330, 64, 4096), (300, 64, 4096), (700, 64, 5632), (700, 128, 5632)])
+@pytest.mark.parametrize("where", ["gate", "up", "down"])
+@pytest.mark.parametrize("value", [np.inf, np.nan, 3.4e38])
+def test_limits_wide_tiles(T, d, F, where, value):
+    test_limits(T, d, F, where, value)
+
+
+def _backward64(x, dout, wg, wu, wd, ids):
+    """dx and the experts' gradients of a top-1 layer (gate weights 1, no
+    router gradient) in float64."""
+    dx = np.zeros(x.shape)
+    dw = []
+    for e in range(len(wg)):
+        t = np.nonzero(ids[:, 0] == e)[0]
+        xe, dy, g, u, d = (a.astype(np.float64) for a in (x[t], dout[t], wg[e], wu[e], wd[e]))
+        g, u, wge, wue = xe @ g, xe @ u, g, u
+        s = 1 / (1 + np.exp(-g))
+        dh = dy @ d.T
+        dg, du = dh * u * (s + g * s * (1 - s)), dh * g * s
+        dx[t] = dg @ wge.T + du @ wue.T
+        dw.append((xe.T @ dg, xe.T @ du, (g * s * u).T @ dy))
+    return dx, *(np.stack(w) for w in zip(*dw))
+
+
+# The weight gradients' tiles at hundreds of rows per expert: 128 x 64 with two
+# wave groups, 128 x 128 with one (512 tiles and more), and both at expert
+# loads that leave part of a round of steps (16 rows, or 32 with two groups).
+@pytest.mark.parametrize("T,d,F,E", [(1000, 256, 1024, 8), (1111, 256, 1024, 8), (2048, 512, 2048, 8), (1777, 512, 2048, 8)])
+def test_weight_gradients(T, d, F, E):
+    layer = mh.Layer(d, F, E, 1)
+    layer.fill_synthetic(13, 0.05, 0.05)
+    x, dout = orc.synth((T, d), 13, 0, 1.0), orc.synth((T, d), 13, 1, 1.0)
+    dxd, ids, out = mh.DeviceArray.from_host(x), mh.DeviceArray((T, 1), np.int32), mh.DeviceArray((T, d))
+    layer.forward_dev(dxd.ptr, T, out.ptr, None, ids.ptr)
+    outs = [mh.DeviceArray(s) for s in ((T, d), (d, E), (E, d, F), (E, d, F), (E, F, d))]
+
+    def run(dout):
+        dod = mh.DeviceArray.from_host(dout)
+        layer.backward_dev(dxd.ptr, T, dod.ptr, 0.0, *[a.ptr for a in outs])
+        mh.synchronize()
+        return [a.to_host() for a in (outs[0], *outs[2:])]
+
+    got = run(dout)
+    w = [np.stack(m) for m in zip(*(layer.get_expert(e) for e in range(E)))]
+    ids = ids.to_host()
+    ref = _backward64(x, dout, *w, ids)
+    for a, b in zip(got, ref):
+        assert orc.rel_l2(a, b) < 3e-6   # (sums of at most 4096 products, as above)
+    # One infinity in dout: its row of dH, dG and dU is infinite, and so are
+    # the sums of the expert's gradients that take it.
+    dout[7, 9] = np.inf
+    bad = run(dout)
+    e = int(ids[7, 0])
+    wg, wu, wd = (m[e].astype(np.float64) for m in w)
+    g, u = x[7].astype(np.float64) @ wg, x[7].astype(np.float64) @ wu
+    s = 1 / (1 + np.exp(-g))
+    sign = np.sign(wd[:, 9])
+    inf = lambda a, b: np.sign(np.outer(a, b)) * np.inf
+    assert np.array_equal(bad[1][e], inf(x[7], sign * u * (s + g * s * (1 - s))))
+    assert np.array_equal(bad[2][e], inf(x[7], sign * g * s))
+    assert np.array_equal(bad[3][e][:, 9], inf(g * s * u, [1.0])[:, 0])
+    assert np.isfinite(np.delete(bad[3][e], 9, 1)).all()
+    for a, b in zip(bad[1:], got[1:]):
+        assert np.array_equal(np.delete(a, e, 0).view(np.uint32), np.delete(b, e, 0).view(np.uint32))
+    layer.close()
