@@ -520,28 +520,43 @@ __global__ __launch_bounds__(256 * KG, 2) void reduce_split_kernel(ReduceGemm g,
     }
     // Sums that are not finite, or too small for the split: again as float
     // products (gemm_split.h), rows r + lh at a time.
+    SumCheck check;
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int j = 0; j < WN; ++j) {
-            if (!any_float_sum(acc[i][j])) continue;
-            const float *ca = g.a + m0 + (wm * WM + i) * 32 + li;
-            const float *cb = g.b + n0 + (wn * WN + j) * 32 + li;
-            fx16 f;
+        for (int j = 0; j < WN; ++j) check.add(acc[i][j]);
+    bool fits = check.fits();
+    if (!fits) {
+        SmallCheck small;
 #pragma unroll
-            for (int q = 0; q < 16; ++q) f[q] = 0.f;
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j) small.add(acc[i][j]);
+        fits = small.fits(check);
+    }
+    if (!fits) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                const float *ca = g.a + m0 + (wm * WM + i) * 32 + li;
+                const float *cb = g.b + n0 + (wn * WN + j) * 32 + li;
+                fx16 f;
+#pragma unroll
+                for (int q = 0; q < 16; ++q) f[q] = 0.f;
 #pragma unroll 1
-            for (int r = r0; r < r1; r += 2) {
-                const int row = min(r + lh, r1 - 1);
-                float x = ca[(GATHER ? token(g.perm[row]) : (size_t)row) * g.lda];
-                float y = cb[(size_t)row * g.ldb];
-                if (r + lh >= r1) x = y = 0.f;
-                f = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, f, 0, 0, 0);
-            }
+                for (int r = r0; r < r1; r += 2) {
+                    const int row = min(r + lh, r1 - 1);
+                    float x = ca[(GATHER ? token(g.perm[row]) : (size_t)row) * g.lda];
+                    float y = cb[(size_t)row * g.ldb];
+                    if (r + lh >= r1) x = y = 0.f;
+                    f = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, f, 0, 0, 0);
+                }
 #pragma unroll
-            for (int q = 0; q < 16; ++q)
-                acc[i][j][q] = float_sum_needed(acc[i][j][q]) ? f[q] : acc[i][j][q];
-        }
+                for (int q = 0; q < 16; ++q)
+                    acc[i][j][q] = float_sum_needed(acc[i][j][q]) ? f[q] : acc[i][j][q];
+            }
+    }
     // Lane l, register q of a block: row 8 (q / 4) + 4 (l / 32) + q % 4,
     // column l % 32.
 #pragma unroll

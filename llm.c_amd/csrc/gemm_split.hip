@@ -19,6 +19,13 @@ constexpr int BM = kGemmBM;   // 128
 constexpr int KT = 32;        // reduction granularity of splits and pieces
 constexpr int kThreads = 256;
 
+__device__ __forceinline__ bool any_float_sum(fx16 a) {
+    bool any = false;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) any |= float_sum_needed(a[r]);
+    return __ballot(any) != 0;
+}
+
 // One tile (m-tile mtg, n-tile nt) over the nk 32-wide K slices from element
 // kb; WM x WN waves, operands loaded D steps ahead.  The down projection writes its partial to slot `slot` (c + slot *
 // split_stride) and, with npieces > 0, records npieces for the tile's rows.
