@@ -376,7 +376,17 @@ __global__ __launch_bounds__(256) void reduce_gemm_kernel(ReduceGemm g) {
 // 113; on the fp32 MFMAs 348 and 169.
 constexpr int kRedAhead = 4;
 
-template <bool GATHER, int WM, int WN, int KG>
+// SHORT: loads wholly past the expert's range are left out.  With few rows
+// most of the first five are, and a load costs the same there (the gathered
+// ones wait for perm one after another).  Up to kRedShortRows rows per expert
+// on average; where most loads are in range the branches cost more.  Whole
+// backward, us without and with: 6 rows (T = 71, d = 192, F = 128, E = 12,
+// top-3) 96.5, 93.0; 12 (T = 200, d = 1024, F = 512, E = 64, top-4) 593, 587;
+// 14 (T = 210, d = 320, F = 256, E = 15) 126.9, 119.0; 31 665.7, 664.1; 62 775.8,
+// 783.9.
+constexpr int kRedShortRows = 32;
+
+template <bool GATHER, int WM, int WN, int KG, bool SHORT>
 __global__ __launch_bounds__(256 * KG, 2) void reduce_split_kernel(ReduceGemm g, unsigned topk_magic,
                                                                 unsigned topk_one) {
     using namespace split;
@@ -419,6 +429,13 @@ __global__ __launch_bounds__(256 * KG, 2) void reduce_split_kernel(ReduceGemm g,
             rb[S][i] = qb[(unsigned)lane];
         }
         load_pix(r + SR);
+    };
+    auto load_in = [&](auto set, int r) {
+        constexpr int S = decltype(set)::value;
+        if (!SHORT || r < r1) load(set, r);
+        else
+#pragma unroll
+            for (int i = 0; i < 8; ++i) ra[S][i] = rb[S][i] = 0.f;
     };
     // Mask: rows past the range count as zeros.
     auto store = [&](auto set, auto mask, int buf, int r) {
@@ -472,7 +489,7 @@ __global__ __launch_bounds__(256 * KG, 2) void reduce_split_kernel(ReduceGemm g,
                 for (int j = 0; j < WN; ++j)
                     acc[i][j] = mma(fa[i][kPairA[q]], fb[j][kPairB[q]], acc[i][j]);
         store(Next{}, mask, buf ^ 1, r + SR);
-        load(Next{}, r + SR * (D + 1));
+        load_in(Next{}, r + SR * (D + 1));
         __syncthreads();
     };
     if (r0 < r1) {
@@ -486,12 +503,12 @@ __global__ __launch_bounds__(256 * KG, 2) void reduce_split_kernel(ReduceGemm g,
         // (the group's own rows: step i at r + 16 kg)
         const int o = 16 * kg;
         load_pix(r0 + o);
-        load(S0{}, r0 + o);
-        load(S1{}, r0 + o + SR);
-        load(S2{}, r0 + o + 2 * SR);
-        load(S3{}, r0 + o + 3 * SR);
+        load_in(S0{}, r0 + o);
+        load_in(S1{}, r0 + o + SR);
+        load_in(S2{}, r0 + o + 2 * SR);
+        load_in(S3{}, r0 + o + 3 * SR);
         store(S0{}, Mask{}, 0, r0 + o);
-        load(S0{}, r0 + o + 4 * SR);
+        load_in(S0{}, r0 + o + 4 * SR);
         __syncthreads();
         int r = r0;
         for (; r + 5 * SR <= r1; r += 4 * SR) {   // (the rows stored are all there)
@@ -1044,18 +1061,23 @@ hipError_t launch_moe_backward(const BackwardArgs &b, hipStream_t s) {
             // perm < T k <= 2^31 / 64 and k <= 16), or perm itself for k = 1.
             const unsigned magic = k > 1 ? (unsigned)((((unsigned long long)1 << 32) + k - 1) / k) : 0;
             const unsigned one = k > 1 ? 0u : ~0u;
+            using I1 = std::integral_constant<int, 1>;
+            using I2 = std::integral_constant<int, 2>;
             auto go = [&](auto wm, auto wn) {
                 constexpr int WM = decltype(wm)::value, WN = decltype(wn)::value;
                 const dim3 grid((unsigned)(N / (64 * WN)), (unsigned)(M / (64 * WM)), (unsigned)E);
-                if (tiles(WM, WN) < 2 * cus)
-                    hipLaunchKernelGGL((reduce_split_kernel<decltype(gather)::value, WM, WN, 2>),
-                                       grid, dim3(512), 0, s, g, magic, one);
-                else
-                    hipLaunchKernelGGL((reduce_split_kernel<decltype(gather)::value, WM, WN, 1>),
-                                       grid, dim3(256), 0, s, g, magic, one);
+                auto launch = [&](auto kg, auto few) {
+                    constexpr int KG = decltype(kg)::value;
+                    hipLaunchKernelGGL((reduce_split_kernel<decltype(gather)::value, WM, WN, KG,
+                                                            decltype(few)::value>),
+                                       grid, dim3(256 * KG), 0, s, g, magic, one);
+                };
+                const bool two = tiles(WM, WN) < 2 * cus, few = n < (size_t)kRedShortRows * E;
+                if (few && two) launch(I2{}, T_{});
+                else if (few)   launch(I1{}, T_{});
+                else if (two)   launch(I2{}, F_{});
+                else            launch(I1{}, F_{});
             };
-            using I1 = std::integral_constant<int, 1>;
-            using I2 = std::integral_constant<int, 2>;
             if (M % 128 == 0 && N % 128 == 0 && tiles(2, 2) >= cus) go(I2{}, I2{});
             else if (M % 128 == 0 && tiles(2, 1) >= cus)           go(I2{}, I1{});
             else if (N % 128 == 0 && tiles(1, 2) >= cus)           go(I1{}, I2{});

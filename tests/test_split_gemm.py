@@ -309,3 +309,25 @@ def test_weight_gradients(T, d, F, E):
     for a, b in zip(bad[1:], got[1:]):
         assert np.array_equal(np.delete(a, e, 0).view(np.uint32), np.delete(b, e, 0).view(np.uint32))
     layer.close()
+
+
+# Experts with few rows (none, one, and up to a few steps of 16 past what the
+# short form's mean allows), on every tile: 64 x 64, 128 x 64 (both widths),
+# 128 x 128, with one and two wave groups.
+@pytest.mark.parametrize("d,F,E", [(64, 64, 5), (192, 128, 12), (128, 448, 60), (448, 128, 60), (256, 1024, 20), (512, 512, 40)])
+@pytest.mark.parametrize("T", [1, 17, 100])
+def test_weight_gradients_few_rows(T, d, F, E):
+    layer = mh.Layer(d, F, E, 1)
+    layer.fill_synthetic(15, 0.3, 0.05)
+    layer.set_bias((3.0 * np.cos(np.arange(E))).astype(np.float32))   # (uneven loads)
+    x, dout = orc.synth((T, d), 15, 0, 1.0), orc.synth((T, d), 15, 1, 1.0)
+    dxd, dod, ids, out = mh.DeviceArray.from_host(x), mh.DeviceArray.from_host(dout), mh.DeviceArray((T, 1), np.int32), mh.DeviceArray((T, d))
+    layer.forward_dev(dxd.ptr, T, out.ptr, None, ids.ptr)
+    outs = [mh.DeviceArray(s) for s in ((T, d), (d, E), (E, d, F), (E, d, F), (E, F, d))]
+    layer.backward_dev(dxd.ptr, T, dod.ptr, 0.0, *[a.ptr for a in outs])
+    mh.synchronize()
+    w = [np.stack(m) for m in zip(*(layer.get_expert(e) for e in range(E)))]
+    ref = _backward64(x, dout, *w, ids.to_host())
+    for a, b in zip((outs[0], *outs[2:]), ref):
+        assert orc.rel_l2(a.to_host(), b) < 3e-6   # (as in test_weight_gradients)
+    layer.close()
