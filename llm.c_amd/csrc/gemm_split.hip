@@ -486,12 +486,17 @@ GemmPlan gemm_plan(int N, int K, int max_mtiles, bool allow_split) {
             p.ksplit *= 2;
         return p;
     }
-    // Without a split: 256-column tiles (each column split once per 128
-    // rows) while they make half a workgroup per CU, 128-column ones (split
-    // by both wave rows) down to 64 workgroups, 64-column ones below.
+    // Without a split: 256-column tiles (each column split once per 128 rows)
+    // while there is one for every CU, 128-column ones (split by both wave
+    // rows) down to a quarter, 64-column ones below.  256 columns from half a
+    // tile per CU on against one, us per layer: d = 512, F = 2048, E = 4, top-2 T
+    // = 256 88.8 / 75.9; d = 2048, F = 1024, E = 16, top-4 T = 200 197.1 / 151.2; d
+    // = 2048, F = 8192, E = 2 T = 64 188.0 / 140.0 (one and a half per CU: even).
+    // 128 columns from an eighth or half on: within 2 % either way.
     auto tiles = [&](int bn) { return (long)max_mtiles * ((N + bn - 1) / bn); };
-    if (p.bn > 128 && tiles(256) < 128) p.bn = 128;
-    if (p.bn > 64 && tiles(p.bn) * (p.bn / 64) < 128) p.bn = 64;
+    const long cus = device_cus();
+    if (p.bn > 128 && tiles(256) < cus) p.bn = 128;
+    if (p.bn == 128 && tiles(128) < cus / 4) p.bn = 64;
     return p;
 }
 

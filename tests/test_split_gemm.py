@@ -244,7 +244,7 @@ def test_wide_tiles_past_the_width(T, d, F, E, k):
 
 # gate/up on 256-column tiles (one wave for 128 rows, last m-tiles of one to
 # four 32-row blocks), without and with a split tail (2 and 4 pieces).
-@pytest.mark.parametrize("T,d,F", [(330, 64, 4096), (300, 64, 4096), (700, 64, 5632), (700, 128, 5632)])
+@pytest.mark.parametrize("T,d,F", [(330, 64, 6656), (300, 64, 6656), (700, 64, 5632), (700, 128, 5632)])
 @pytest.mark.parametrize("where", ["gate", "up", "down"])
 @pytest.mark.parametrize("value", [np.inf, np.nan, 3.4e38])
 def test_limits_wide_tiles(T, d, F, where, value):
