@@ -53,9 +53,13 @@ struct DispatchArgs {
 };
 
 // Up to this many (token, slot) assignments, and router workgroups, the
-// router's last workgroup performs the dispatch itself.  (One workgroup sorts
-// 512 as fast as a launch of their own, 1024 about 4 us faster; at 3009 the
-// layer of T = 1003, d = 320, top-3 takes 108.8 us fused, 100.7 apart.)
+// router's last workgroup performs the dispatch itself.  Up to 1024 one
+// workgroup sorts as fast as a launch of their own (within 1.5 us either way:
+// 400 to 1024 assignments of seven layers), past it the launch is faster: us
+// per layer fused and apart, d = 256, F = 1024, E = 8, top-2 T = 600 54.2 / 52.3,
+// 1500 74.4 / 64.1, 2048 101.1 / 85.8; d = 1024, F = 512, E = 64, top-8 T = 200
+// 149.0 / 149.7, 400 169.5 / 165.2; d = 512, F = 1024, E = 64, top-1 T = 1500
+// 134.3 / 130.5.
 constexpr int kFusedDispatchMax = 1024;
 constexpr int kFusedDispatchMaxBlocks = 16;
 
