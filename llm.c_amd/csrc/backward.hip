@@ -934,9 +934,9 @@ size_t backward_tail_floats(int d, int F, int max_mtiles, int E) {
     return (size_t)g * kGemmBM * 256;
 }
 
-int backward_slot_splits(int d, int F, int max_mtiles, size_t n) {
+int backward_slot_splits(int d, int F, int max_mtiles, size_t n, int k) {
     if (!backward_engine_ok(d, F)) return 1;
-    return std::max(down_plan(d, F, max_mtiles, n).slots, down_plan(d, 2 * F, max_mtiles, n).slots);
+    return std::max(down_plan(d, F, max_mtiles, n, k).slots, down_plan(d, 2 * F, max_mtiles, n, k).slots);
 }
 
 hipError_t launch_moe_backward(const BackwardArgs &b, hipStream_t s) {
@@ -983,11 +983,11 @@ hipError_t launch_moe_backward(const BackwardArgs &b, hipStream_t s) {
         // (Y and dX: down-projection shapes, by slot with split partials or
         // stream-K pieces, moe::down_plan; one piece-count table serves both
         // in turn.)
-        const DownPlan py = down_plan(d, F, b.max_mtiles, n);
+        const DownPlan py = down_plan(d, F, b.max_mtiles, n, k);
         GemmArgs gy = g;
         gy.a = b.H; gy.b = b.wdT; gy.c = b.Y; gy.K = F; gy.N = d; gy.ldc = d;
         gy.ksplit = py.slots; gy.split_stride = nd;
-        gy.streamk = py.streamk; gy.sk_groups = py.groups; gy.sk_bn = py.bn; gy.pieces = b.pieces;
+        gy.streamk = py.streamk; gy.sk_groups = py.groups; gy.bn = py.bn; gy.pieces = b.pieces;
         BWD_TRY(launch_gemm_down(gy, s));
         hipLaunchKernelGGL(slot_kernel, dim3(slot_grid), dim3(256), 0, s,
                            SlotRows{b.Y, 1, py.slots, nd, py.streamk ? b.pieces : nullptr, py.bn},
@@ -1001,11 +1001,11 @@ hipError_t launch_moe_backward(const BackwardArgs &b, hipStream_t s) {
         }
         BWD_TRY(launch_gemm_bwd(gh, 3, s));
         BWD_TRY(launch_tail_fixup(gh, 3, s));
-        const DownPlan px = down_plan(d, 2 * F, b.max_mtiles, n);
+        const DownPlan px = down_plan(d, 2 * F, b.max_mtiles, n, k);
         GemmArgs gx = g;
         gx.a = GU; gx.b = b.wguT; gx.c = b.Y; gx.K = 2 * F; gx.N = d; gx.ldc = d;
         gx.ksplit = px.slots; gx.split_stride = nd;
-        gx.streamk = px.streamk; gx.sk_groups = px.groups; gx.sk_bn = px.bn; gx.pieces = b.pieces;
+        gx.streamk = px.streamk; gx.sk_groups = px.groups; gx.bn = px.bn; gx.pieces = b.pieces;
         BWD_TRY(launch_gemm_down(gx, s));
         dXr = SlotRows{b.Y, 1, px.slots, nd, px.streamk ? b.pieces : nullptr, px.bn};
     } else {

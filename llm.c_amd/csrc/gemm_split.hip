@@ -278,8 +278,37 @@ __device__ __forceinline__ TailLayout tail_layout(const GemmArgs &a, int ntiles,
     return TailLayout{live - r, r, sp};
 }
 
+// Down projection in stream-K form: how `grid` workgroups share `tiles` live
+// tiles of nks K slices.  p > 0: every tile in p even pieces, one per
+// workgroup; 0: runs of ceil(tiles nks / grid) slices over the flat list of
+// (tile, slice) units, most of which touch two tiles.
+// Runs load every workgroup alike, but a second tile is a second prologue
+// and epilogue, about kSkPass slices' time; so they are taken where even
+// pieces would be longer than a run by more than that (T = 4096, d = 256, F =
+// 1024, E = 8, top-2: three pieces of 11 slices 111.0 us per layer, runs of 9
+// 119.1; T = 139, d = 576, F = 7072, E = 22, top-4: four pieces of 56 slices 297,
+// runs of 50 283).
+// A piece has four slices or so: fewer cost more in partials than they save
+// (T = 59, d = 192, F = 896, E = 7, top-4: 14 pieces 44.2 us, 7 37.7), and the
+// combine adds a tile's pieces for each of a token's k slots, eight loads at a
+// time: 64 in all at most (T = 24, d = 256, F = 3200, E = 8, top-6: 25 pieces
+// 79.3 us, 10 54.0).
+constexpr int kSkPass = 2;
+__host__ __device__ constexpr int sk_max_pieces(int nks, int topk) {
+    const int c = topk < 8 ? 64 / topk : 8, l = (nks + 3) / 4;
+    return c < l ? c : l;
+}
+__host__ __device__ constexpr int sk_even_pieces(int tiles, int nks, int grid, int topk) {
+    const int room = tiles > 0 ? grid / tiles : 0, most = sk_max_pieces(nks, topk);
+    if (room > most) return most;
+    if (room < 1) return 0;
+    const int run = (int)(((long)tiles * nks + grid - 1) / grid);
+    return (nks + room - 1) / room - run > kSkPass ? 0 : room;
+}
+
 // Grid: the (m-tile, n-tile) pairs, times the reduction splits.  Down
-// projection in stream-K form (a.streamk): workgroup g takes units
+// projection in stream-K form (a.streamk): a piece of a tile each
+// (sk_even_pieces), or workgroup g takes units
 // [g per, (g + 1) per) of the flat list of (live tile, K slice) units, per =
 // ceil(units / grid); each tile it touches is a piece whose index within
 // the tile (0 for the workgroup holding the tile's first slice) is the
@@ -293,7 +322,16 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_kernel(GemmArgs a) {
     const int ntiles = (a.N + BN - 1) / BN;
     const int nks = a.K / KT;
     if (MODE == 1 && a.streamk) {
-        const long units = (long)a.tile_off[a.E] * ntiles * nks;
+        const int tiles = a.tile_off[a.E] * ntiles;
+        if (const int p = sk_even_pieces(tiles, nks, gridDim.x, a.topk)) {
+            const int tile = blockIdx.x / p, i = blockIdx.x - tile * p;
+            if (tile >= tiles) return;
+            const int k0 = i * nks / p, k1 = (i + 1) * nks / p;
+            gemm_tile<MODE, WM, WN>(a, smem, tile / ntiles, tile % ntiles, k0 * KT, k1 - k0, i,
+                                    i == 0 ? p : 0);
+            return;
+        }
+        const long units = (long)tiles * nks;
         const long per = (units + gridDim.x - 1) / gridDim.x;
         long u = (long)blockIdx.x * per;
         const long uend = u + per < units ? u + per : units;
@@ -355,17 +393,17 @@ hipError_t launch_grouped(const GemmArgs &a, hipStream_t s) {
 
 template <int MODE>
 hipError_t launch_mode(const GemmArgs &a, hipStream_t s) {
-    const GemmPlan pl = gemm_plan(a.N, a.K, a.max_mtiles, MODE == 1);
+    const int bn = MODE == 1 ? a.bn : gemm_plan(a.N, a.K, a.max_mtiles, false).bn;
     if (a.K % KT || a.N % 64) return hipErrorInvalidValue;
     if (MODE == 1 && a.streamk) {
         if (!a.pieces || a.sk_groups <= 0) return hipErrorInvalidValue;
-        if (a.sk_bn == 128) return launch_grouped<MODE, 2, 2>(a, s);
+        if (bn == 128) return launch_grouped<MODE, 2, 2>(a, s);
         return hipErrorInvalidValue;
     }
     if (a.ksplit < 1 || (a.K / KT) % a.ksplit || (MODE != 1 && a.ksplit != 1)) return hipErrorInvalidValue;
-    if (MODE != 1 && a.tail_groups > 0 && (!a.tail_part || a.N % 256 || pl.bn != 256))
+    if (MODE != 1 && a.tail_groups > 0 && (!a.tail_part || a.N % 256 || bn != 256))
         return hipErrorInvalidValue;
-    switch (pl.bn) {
+    switch (bn) {
         case 256: return launch_grouped<MODE, 1, 4>(a, s);
         case 128: return launch_grouped<MODE, 2, 2>(a, s);
         case 64:  return launch_grouped<MODE, 4, 1>(a, s);
@@ -505,7 +543,7 @@ GemmPlan gemm_plan(int N, int K, int max_mtiles, bool allow_split) {
 // 4096, d = 256, F = 1024, E = 8: 115.8 us per layer against 121; 256 columns
 // over two per CU 126.5, 128 over four 132).
 constexpr int kSkBN = 128, kSkPerCu = 2;
-DownPlan down_plan(int N, int K, int max_mtiles, size_t n) {
+DownPlan down_plan(int N, int K, int max_mtiles, size_t n, int k) {
     const GemmPlan g = gemm_plan(N, K, max_mtiles, true);
     DownPlan p{g.bn, g.ksplit, 0, 0};
     if (g.bn < 128 || K % KT) return p;
@@ -514,23 +552,30 @@ DownPlan down_plan(int N, int K, int max_mtiles, size_t n) {
     // (or tiles split a fixed 2 or 4 ways) leave a partial last round.
     const long cus = device_cus();
     if ((long)max_mtiles * ((N + 255) / 256) >= 8 * cus) return p;
-    const long nks = K / KT;
-    // The fewest live tiles n rows can make (all rows in full m-tiles) set
-    // the shortest run per workgroup, hence the most pieces a tile can have.
-    const long tiles_min = (long)((n + BM - 1) / BM) * ((N + kSkBN - 1) / kSkBN);
-    const long units_min = tiles_min * nks;
-    // At least 4 slices per workgroup on small problems, counted on the most
-    // tiles the rows can make: few rows over many experts make an m-tile each
-    // (T = 15, d = 192, F = 4768, E = 170, top-7: counted on the fewest, 74
-    // workgroups did the work of 160 tiles).  The partials stay bounded:
-    // slots n N is about groups tiles at most.
-    const long units_max = (long)max_mtiles * ((N + kSkBN - 1) / kSkBN) * nks;
-    const long groups = std::max(1L, std::min(kSkPerCu * cus, units_max / 4));
-    const long per_min = (units_min + groups - 1) / groups;
+    const long nks = K / KT, tn = (N + kSkBN - 1) / kSkBN;
+    // As many workgroups as the most tiles the rows can make have pieces (few rows over many experts make an m-tile each: T = 15, d =
+    // 192, F = 4768, E = 170, top-7: counted on the fewest, 74 workgroups did
+    // the work of 160 tiles).
+    const long tiles_max = max_mtiles * tn;
+    const int most = sk_max_pieces((int)nks, k);
+    const long groups = std::max(1L, std::min(kSkPerCu * cus, tiles_max * most));
+    // Too short to split: whole tiles, no piece counts (T = 60, d = 192, F =
+    // 96, E = 30, top-6: 44.4 -> 35.3 us).
+    if (most == 1 && tiles_max <= groups) {
+        p.bn = gemm_plan(N, K, max_mtiles, false).bn;
+        return p;
+    }
+    // The fewest live tiles n rows can make (all rows in full m-tiles) have
+    // the most pieces: `most` or the workgroups there are for each, and where
+    // these are at most `most`, runs of a `most + 1`-th of a tile and more.
+    // The partials stay bounded: slots n N is about groups tiles at most.
+    const long tiles_min = (long)((n + BM - 1) / BM) * tn;
+    const long per_min = (tiles_min * nks + groups - 1) / groups;
+    const long run_slots = std::min((nks - 1 + per_min - 1) / per_min + 1, (long)most + 2);
     p.bn = kSkBN;
     p.streamk = 1;
     p.groups = (int)groups;
-    p.slots = (int)((nks - 1 + per_min - 1) / per_min + 1);
+    p.slots = (int)std::max(run_slots, std::min(groups / tiles_min, (long)most));
     return p;
 }
 

@@ -1237,10 +1237,10 @@ struct FwdPlan {
     bool use_decode = false, fused = false;
     bool tiny = false;      // a step of at most moe::kTinySlots assignments (decode_tiny.hip)
     int ksplit = 1;         // partial products per slot the combine adds (at most, stream-K)
-    int streamk = 0, sk_groups = 0, sk_bn = 0;   // down projection in stream-K form (moe::down_plan)
+    int streamk = 0, sk_groups = 0, down_bn = 0;   // down projection in stream-K form (moe::down_plan)
     size_t h_floats = 0;    // H [n x F] (grouped GEMMs, unfused decode)
     size_t ys_floats = 0;   // per-slot products / split-K partials
-    size_t pieces_ints = 0; // stream-K piece counts [n][ceil(d / sk_bn)]
+    size_t pieces_ints = 0; // stream-K piece counts [n][ceil(d / down_bn)]
     int gu_tail = 0;        // gate/up split tail: workgroups per round (moe::gateup_tail_groups)
     size_t gu_part_floats = 0;  // its pieces
     size_t order_ints = 0;  // the down projection's short-first m-tile order (whole tiles, >= 4 rounds)
@@ -1254,7 +1254,7 @@ struct FwdBufs {
     int *counts = nullptr, *offsets = nullptr, *tile_off = nullptr, *tile_expert = nullptr;
     int *perm = nullptr;    // [n]
     float *h = nullptr, *ys = nullptr;
-    int *pieces = nullptr;     // [n][ceil(d / sk_bn)] (stream-K down projection)
+    int *pieces = nullptr;     // [n][ceil(d / down_bn)] (stream-K down projection)
     float *gu_part = nullptr;  // gate/up split-tail pieces
     int *order = nullptr;      // [max_mtiles] m-tile order of the down projection
     int *counters = nullptr;   // kMaxCounters ints, zero between launches
@@ -1310,12 +1310,12 @@ int plan_level(const MoeHipLayer *L, int T, FwdPlan *p, bool probs_given, int le
     } else {
         // Small grids split the down projection's reduction (a fixed split,
         // or stream-K pieces); the combine adds the partials in order.
-        moe::DownPlan dp = moe::down_plan(d, F, p->max_mtiles, n);
+        moe::DownPlan dp = moe::down_plan(d, F, p->max_mtiles, n, k);
         if (lean >= 2) dp = moe::DownPlan{moe::gemm_plan(d, F, p->max_mtiles, true).bn, 1, 0, 0};
         p->ksplit = dp.slots;
         p->streamk = dp.streamk;
         p->sk_groups = dp.groups;
-        p->sk_bn = dp.bn;
+        p->down_bn = dp.bn;
         p->pieces_ints = dp.streamk ? n * (size_t)((d + dp.bn - 1) / dp.bn) : 0;
         p->gu_tail = lean ? 0 : moe::gateup_tail_groups(2 * F, d, p->max_mtiles, E);
         p->gu_part_floats = (size_t)p->gu_tail * moe::kGemmBM * 256;
@@ -1513,7 +1513,7 @@ static int run_forward(MoeHipLayer *L, const float *x, int T, float *out, float 
         dn.split_stride = n * (size_t)d;
         dn.streamk = p.streamk;
         dn.sk_groups = p.sk_groups;
-        dn.sk_bn = p.sk_bn;
+        dn.bn = p.down_bn;
         dn.pieces = b.pieces;
         if (b.order) {
             // The experts' short last m-tiles first: a CU that finishes one of
@@ -1528,7 +1528,7 @@ static int run_forward(MoeHipLayer *L, const float *x, int T, float *out, float 
     moe::CombineArgs ca{b.ys, b.gw, out, T, d, k, accumulate, p.ksplit, n * (size_t)d};
     if (p.streamk) {
         ca.pieces = b.pieces;
-        ca.pieces_cols = p.sk_bn;
+        ca.pieces_cols = p.down_bn;
     }
     HIP_TRY(moe::launch_combine(ca, s));
     if (g_timing) {
@@ -1747,7 +1747,7 @@ int moe_hip_backward_dev(MoeHipLayer *L, const float *x, int T, const float *dou
     // gradient's chunk partials reuse it]; Y [splits][n x d], dY [n x d];
     // dgw, inv [n]; dlogits [T x E].
     const size_t nF = n * F, nd = n * d, ndh = moe::backward_dh_floats(n, d, F, E);
-    const size_t ysplits = (size_t)moe::backward_slot_splits(d, F, max_mtiles, n);
+    const size_t ysplits = (size_t)moe::backward_slot_splits(d, F, max_mtiles, n, k);
     const size_t npieces = engine ? n * (size_t)((d + 127) / 128) : 0;
     const size_t ntail = moe::backward_tail_floats(d, F, max_mtiles, E);
     // (the split-tail pieces last, 256-byte aligned)

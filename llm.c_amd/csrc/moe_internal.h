@@ -87,7 +87,7 @@ struct GemmArgs {
     // s, and pieces[row][n-tile] receives the tile's piece count.
     int streamk = 0;
     int sk_groups = 0;
-    int sk_bn = 0;       // its tile width (DownPlan::bn)
+    int bn = 0;          // the down projection's tile width (DownPlan::bn)
     int *pieces = nullptr;
     // Backward epilogues: mode 2 also writes H = swiglu(G, U) to c2.
     float *c2 = nullptr;
@@ -279,7 +279,7 @@ hipError_t launch_moe_backward(const BackwardArgs &b, hipStream_t s);
 bool backward_engine_ok(int d, int F);
 // Partial products per slot row the engine path leaves in Y (1 otherwise);
 // n = T * k.
-int backward_slot_splits(int d, int F, int max_mtiles, size_t n);
+int backward_slot_splits(int d, int F, int max_mtiles, size_t n, int k);
 // Floats of BackwardArgs::tail_part the engine path uses (0: none).
 size_t backward_tail_floats(int d, int F, int max_mtiles, int E);
 // Floats of BackwardArgs::dH: n x F, and at least one row chunk of the
@@ -317,11 +317,11 @@ GemmPlan gemm_plan(int N, int K, int max_mtiles, bool allow_split);
 
 // The forward's down projection: classic (the gemm_plan split) or, for
 // grids of a few rounds, stream-K over `groups` workgroups with at most
-// `slots` partials per tile.  n: the routed rows (T * k).
+// `slots` partials per tile.  n: the routed rows (T * k), k: slots per token.
 struct DownPlan {
     int bn, slots, streamk, groups;
 };
-DownPlan down_plan(int N, int K, int max_mtiles, size_t n);
+DownPlan down_plan(int N, int K, int max_mtiles, size_t n, int k);
 // Workgroups per round for a gate/up launch with a split tail (the CUs), or
 // 0 for whole tiles only: used when 256-column tiles make between one and
 // eight per CU, where the last, partial round is a large share of the launch.
