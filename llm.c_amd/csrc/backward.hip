@@ -542,16 +542,7 @@ __global__ __launch_bounds__(256 * KG, 2) void reduce_split_kernel(ReduceGemm g,
     for (int i = 0; i < WM; ++i)
 #pragma unroll
         for (int j = 0; j < WN; ++j) check.add(acc[i][j]);
-    bool fits = check.fits();
-    if (!fits) {
-        SmallCheck small;
-#pragma unroll
-        for (int i = 0; i < WM; ++i)
-#pragma unroll
-            for (int j = 0; j < WN; ++j) small.add(acc[i][j]);
-        fits = small.fits(check);
-    }
-    if (!fits) {
+    if (!check.fits()) {
 #pragma unroll
         for (int i = 0; i < WM; ++i)
 #pragma unroll

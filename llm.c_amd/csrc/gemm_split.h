@@ -94,31 +94,22 @@ __device__ __forceinline__ bool float_sum_needed(float s) {
     return !(fabsf(s) >= kSmallSum && fabsf(s) <= 0x1.fffffep127f) && s != 0.0f;
 }
 
-// Whether a wave has such sums, the cheap answer first: chk stays 0 while they
-// are finite, lo is the smallest magnitude, zeros included (three VALU
-// instructions for two sums; asking each sum the question above cost the weight
-// gradients of T = 1000, d = 1024, F = 512, E = 64, top-4 10 us of 745).
+// Whether a wave has such sums: chk stays 0 while they are finite, lo is the
+// smallest 2 |bits| - 1, the largest number for a zero (five VALU instructions
+// for two sums; asking each sum the question above cost the backward of T =
+// 1000, d = 1024, F = 512, E = 64, top-4 10 us of 770).
 struct SumCheck {
-    float chk = 0.0f, lo = 1.0f;
+    float chk = 0.0f;
+    unsigned lo = ~0u;
     __device__ __forceinline__ void add(fx16 a) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             chk = fmaf(a[r], 0.0f, chk);
-            lo = fminf(lo, fabsf(a[r]));
+            lo = min(lo, (__float_as_uint(a[r]) << 1) - 1u);
         }
     }
-    __device__ __forceinline__ bool fits() const { return !__ballot(!(chk == 0.0f && lo >= kSmallSum)); }
-};
-// Where that does not settle it: the smallest magnitude without the zeros
-// (2 |bits| - 1 is the largest for them).
-struct SmallCheck {
-    unsigned lo = ~0u;
-    __device__ __forceinline__ void add(fx16 a) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) lo = min(lo, (__float_as_uint(a[r]) << 1) - 1u);
-    }
-    __device__ __forceinline__ bool fits(const SumCheck &c) const {
-        return !__ballot(!(c.chk == 0.0f) || lo < (__float_as_uint(kSmallSum) << 1) - 1u);
+    __device__ __forceinline__ bool fits() const {
+        return !__ballot(!(chk == 0.0f) || lo < (__float_as_uint(kSmallSum) << 1) - 1u);
     }
 };
 

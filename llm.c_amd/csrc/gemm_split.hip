@@ -323,30 +323,36 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_kernel(GemmArgs a) {
     const int nks = a.K / KT;
     if (MODE == 1 && a.streamk) {
         const int tiles = a.tile_off[a.E] * ntiles;
-        if (const int p = sk_even_pieces(tiles, nks, gridDim.x, a.topk)) {
-            const int tile = blockIdx.x / p, i = blockIdx.x - tile * p;
+        const int pieces = sk_even_pieces(tiles, nks, gridDim.x, a.topk), b = blockIdx.x;
+        int tile = 0, k0 = 0, k1 = 0, slot = 0, npieces = pieces;
+        long u = 0, uend = 0, per = 0;
+        if (pieces) {   // (32-bit divisions only: a piece may be a few slices)
+            tile = b / pieces;
             if (tile >= tiles) return;
-            const int k0 = i * nks / p, k1 = (i + 1) * nks / p;
-            gemm_tile<MODE, WM, WN>(a, smem, tile / ntiles, tile % ntiles, k0 * KT, k1 - k0, i,
-                                    i == 0 ? p : 0);
-            return;
+            slot = b - tile * pieces;
+            k0 = slot * nks / pieces;
+            k1 = (slot + 1) * nks / pieces;
+        } else {
+            const long units = (long)tiles * nks;
+            per = (units + gridDim.x - 1) / gridDim.x;
+            u = b * per;
+            uend = u + per < units ? u + per : units;
         }
-        const long units = (long)tiles * nks;
-        const long per = (units + gridDim.x - 1) / gridDim.x;
-        long u = (long)blockIdx.x * per;
-        const long uend = u + per < units ? u + per : units;
-        while (u < uend) {
-            const int tile = (int)(u / nks);
-            const int k0 = (int)(u - (long)tile * nks);
-            const int k1 = (int)(k0 + (uend - u) < nks ? k0 + (uend - u) : nks);
-            const long tstart = (long)tile * nks;
-            const int first = (int)(tstart / per);   // workgroup of the tile's first slice
-            const int slot = (int)blockIdx.x - first;
-            const int npieces = (int)((tstart + nks - 1) / per) - first + 1;
+        do {
+            if (!pieces) {
+                if (u >= uend) return;
+                tile = (int)(u / nks);
+                k0 = (int)(u - (long)tile * nks);
+                k1 = (int)(k0 + (uend - u) < nks ? k0 + (uend - u) : nks);
+                const long tstart = (long)tile * nks;
+                const int first = (int)(tstart / per);   // workgroup of the tile's first slice
+                slot = b - first;
+                npieces = (int)((tstart + nks - 1) / per) - first + 1;
+                u += k1 - k0;
+            }
             gemm_tile<MODE, WM, WN>(a, smem, tile / ntiles, tile % ntiles, k0 * KT, k1 - k0, slot,
-                                slot == 0 ? npieces : 0);
-            u += k1 - k0;
-        }
+                                    slot == 0 ? npieces : 0);
+        } while (!pieces);
         return;
     }
     if (MODE != 1 && a.tail_groups > 0) {
