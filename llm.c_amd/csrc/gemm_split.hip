@@ -292,14 +292,18 @@ __device__ __forceinline__ TailLayout tail_layout(const GemmArgs &a, int ntiles,
 // (T = 59, d = 192, F = 896, E = 7, top-4: 14 pieces 44.2 us, 7 37.7), and the
 // combine adds a tile's pieces for each of a token's k slots, eight loads at a
 // time: 64 in all at most (T = 24, d = 256, F = 3200, E = 8, top-6: 25 pieces
-// 79.3 us, 10 54.0).
-constexpr int kSkPass = 2;
-__host__ __device__ constexpr int sk_max_pieces(int nks, int topk) {
-    const int c = topk < 8 ? 64 / topk : 8, l = (nks + 3) / 4;
+// 79.3 us, 10 54.0).  Reductions of 6 to 15 slices on few tiles go down to two
+// slices for up to four pieces (T = 118, d = 256, F = 256, E = 1: two pieces 37.0
+// us, four 35.2; backward T = 71, d = 192, F = 128, E = 12, top-3 92.4, 90.7).
+constexpr int kSkPass = 2, kSkFewTiles = 64;
+__host__ __device__ constexpr int sk_max_pieces(int tiles, int nks, int topk) {
+    const int c = topk < 8 ? 64 / topk : 8;
+    int l = (nks + 3) / 4;
+    if (tiles <= kSkFewTiles && nks >= 6 && nks < 16) l = nks < 8 ? nks / 2 : 4;
     return c < l ? c : l;
 }
 __host__ __device__ constexpr int sk_even_pieces(int tiles, int nks, int grid, int topk) {
-    const int room = tiles > 0 ? grid / tiles : 0, most = sk_max_pieces(nks, topk);
+    const int room = tiles > 0 ? grid / tiles : 0, most = sk_max_pieces(tiles, nks, topk);
     if (room > most) return most;
     if (room < 1) return 0;
     const int run = (int)(((long)tiles * nks + grid - 1) / grid);
@@ -563,8 +567,11 @@ DownPlan down_plan(int N, int K, int max_mtiles, size_t n, int k) {
     // 192, F = 4768, E = 170, top-7: counted on the fewest, 74 workgroups did
     // the work of 160 tiles).
     const long tiles_max = max_mtiles * tn;
-    const int most = sk_max_pieces((int)nks, k);
-    const long groups = std::max(1L, std::min(kSkPerCu * cus, tiles_max * most));
+    const long few = std::min(tiles_max, (long)kSkFewTiles);
+    const int most = sk_max_pieces((int)few, (int)nks, k);
+    const long groups = std::max(1L, std::min(kSkPerCu * cus,
+                                              std::max(tiles_max * sk_max_pieces((int)tiles_max, (int)nks, k),
+                                                       few * most)));
     // Too short to split: whole tiles, no piece counts (T = 60, d = 192, F =
     // 96, E = 30, top-6: 44.4 -> 35.3 us).
     if (most == 1 && tiles_max <= groups) {

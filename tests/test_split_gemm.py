@@ -333,10 +333,10 @@ def test_weight_gradients_few_rows(T, d, F, E):
     layer.close()
 
 
-# The down projection's tiles whole (K = 96), in even pieces (two; bounded by
-# the reduction's length; bounded by a token's slots) and in runs that touch
+# The down projection's tiles whole (K = 96), in even pieces (of two slices; of
+# four; bounded by a token's slots) and in runs that touch
 # two tiles (counted on the most and on the fewest tiles).
-@pytest.mark.parametrize("T,d,F,E,k", [(60, 192, 96, 30, 6), (97, 128, 192, 3, 3), (621, 256, 2304, 2, 1), (24, 256, 3200, 8, 6),
+@pytest.mark.parametrize("T,d,F,E,k", [(60, 192, 96, 30, 6), (97, 128, 192, 3, 3), (118, 256, 256, 1, 1), (621, 256, 2304, 2, 1), (24, 256, 3200, 8, 6),
                                        (1500, 512, 512, 4, 2), (900, 640, 1056, 6, 3), (129, 1024, 4096, 1, 1)])
 def test_down_projection_pieces(T, d, F, E, k):
     hw = _layer(d, F, E, k, T)
