@@ -52,7 +52,7 @@ sys.path.insert(0, os.path.join(ROOT, "llm.c_amd"))
 METRIC = "MoE layer tokens/s + % fp32 MFMA peak (prefill); decode tok/s + HBM GB/s"
 PEAK_FP32_MFMA_TFLOPS = 157.3      # MI355X dense fp32 matrix
 # The grouped GEMMs take each fp32 product as six bf16 MFMA products (operands
-# split exactly into three bf16 terms): their bound is a sixth of the dense
+# split into three bf16 terms): their bound is a sixth of the dense
 # bf16 rate.  Fractions of the fp32 MFMA peak can pass 1.
 PEAK_SPLIT_TFLOPS = 2500.0 / 6.0
 PEAK_HBM_GBS = 8000.0              # MI355X HBM3E

@@ -27,8 +27,9 @@ __device__ __forceinline__ bool any_float_sum(fx16 a) {
 }
 
 // One tile (m-tile mtg, n-tile nt) over the nk 32-wide K slices from element
-// kb; WM x WN waves, operands loaded D steps ahead.  The down projection writes its partial to slot `slot` (c + slot *
-// split_stride) and, with npieces > 0, records npieces for the tile's rows.
+// kb; WM x WN waves, operands loaded D steps ahead.  The down projection
+// writes its partial to slot `slot` (c + slot * split_stride) and, with
+// npieces > 0, records npieces for the tile's rows.
 // Every thread of the workgroup calls this together.
 template <int MODE, int WM, int WN>
 __device__ __forceinline__ void gemm_tile(const GemmArgs &a, char *smem, int mtg, int nt, int kb,
@@ -312,9 +313,9 @@ __host__ __device__ constexpr int sk_even_pieces(int tiles, int nks, int grid, i
 
 // Grid: the (m-tile, n-tile) pairs, times the reduction splits.  Down
 // projection in stream-K form (a.streamk): a piece of a tile each
-// (sk_even_pieces), or workgroup g takes units
-// [g per, (g + 1) per) of the flat list of (live tile, K slice) units, per =
-// ceil(units / grid); each tile it touches is a piece whose index within
+// (sk_even_pieces), or workgroup g takes units [g per, (g + 1) per) of the flat
+// list of (live tile, K slice) units, per = ceil(units / grid); each tile it
+// touches is a piece.  A piece's index within
 // the tile (0 for the workgroup holding the tile's first slice) is the
 // partial slot it writes, and piece 0 records the tile's piece count for
 // the combine.  Slots, pieces and counts follow from the live tile count
@@ -551,7 +552,7 @@ GemmPlan gemm_plan(int N, int K, int max_mtiles, bool allow_split) {
 // Stream-K takes 128-column tiles over two workgroups per CU: as many partials
 // per slot as 256-column tiles over one per CU, with twice the waves (T =
 // 4096, d = 256, F = 1024, E = 8: 115.8 us per layer against 121; 256 columns
-// over two per CU 126.5, 128 over four 132).
+// over two per CU 126.5, 128 over four 132; even pieces since, 109.6).
 constexpr int kSkBN = 128, kSkPerCu = 2;
 DownPlan down_plan(int N, int K, int max_mtiles, size_t n, int k) {
     const GemmPlan g = gemm_plan(N, K, max_mtiles, true);
@@ -563,9 +564,10 @@ DownPlan down_plan(int N, int K, int max_mtiles, size_t n, int k) {
     const long cus = device_cus();
     if ((long)max_mtiles * ((N + 255) / 256) >= 8 * cus) return p;
     const long nks = K / KT, tn = (N + kSkBN - 1) / kSkBN;
-    // As many workgroups as the most tiles the rows can make have pieces (few rows over many experts make an m-tile each: T = 15, d =
-    // 192, F = 4768, E = 170, top-7: counted on the fewest, 74 workgroups did
-    // the work of 160 tiles).
+    // As many workgroups as the most tiles the rows can make have pieces (few
+    // rows over many experts make an m-tile each: T = 15, d = 192, F = 4768, E =
+    // 170, top-7: counted on the fewest, 74 workgroups did the work of 160
+    // tiles).
     const long tiles_max = max_mtiles * tn;
     const long few = std::min(tiles_max, (long)kSkFewTiles);
     const int most = sk_max_pieces((int)few, (int)nks, k);

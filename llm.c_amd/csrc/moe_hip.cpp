@@ -1243,7 +1243,7 @@ struct FwdPlan {
     size_t pieces_ints = 0; // stream-K piece counts [n][ceil(d / down_bn)]
     int gu_tail = 0;        // gate/up split tail: workgroups per round (moe::gateup_tail_groups)
     size_t gu_part_floats = 0;  // its pieces
-    size_t order_ints = 0;  // the down projection's short-first m-tile order (whole tiles, >= 4 rounds)
+    size_t order_ints = 0;  // the down projection's short-first m-tile order (whole tiles, >= 8 per CU)
     size_t wide_probs_floats = 0, wide_ints = 0;   // general routing kernels' buffers (WideBufs)
 };
 
